@@ -648,7 +648,7 @@ __global__ __launch_bounds__(kReducedThreads) void k_imu_reduced(Window w) {
 __global__ __launch_bounds__(kFactorThreads) void k_imu_factor(Window w) {
   using namespace sba_tiles;
   __shared__ double PT[(kMaxFree - 1) * 256];         // panel tiles of the current column, transposed
-  __shared__ double sT[256], xt[256], yk[16], rdiag[16];
+  __shared__ double xt[256], yk[16], rdiag[16];
   __shared__ double x[16 * kMaxFree];                 // right-hand side, then y, then the step (padded by tiles)
   __shared__ unsigned char nz[kMaxFree * kMaxFree];  // nz[i * nb + j], i >= j: tile (i, j) of L is not zero
   __shared__ int rows[kMaxFree];
@@ -681,7 +681,7 @@ __global__ __launch_bounds__(kFactorThreads) void k_imu_factor(Window w) {
       double4v t;
 #pragma unroll
       for (int v = 0; v < 4; ++v) t[v] = D[64 * v + lane];
-      const bool pos = factor_tile(t, sT, xt, rdiag, lane);
+      const bool pos = factor_tile(t, xt, rdiag, lane);
       wave_lds_sync();
 #pragma unroll
       for (int v = 0; v < 4; ++v) D[64 * v + lane] = xt[64 * v + lane];

@@ -850,7 +850,6 @@ __global__ __launch_bounds__(kFactorThreads) void k_factor(Batch b, double* dbg_
   __shared__ double du[256];   // diag(U)
   __shared__ double idg[256];  // 1 / L_ii
   __shared__ double red[32];
-  __shared__ double sT[256];          // the diagonal tile being factored
   __shared__ double sDg[kFT * 256];   // diagonal tiles (wavefront 0), row-major
   __shared__ double sXT[kFT * 256];   // X_KK^T of every tile column
   __shared__ double sP[kFT * 256];    // panel tiles U_KI of the current tile column
@@ -949,7 +948,7 @@ __global__ __launch_bounds__(kFactorThreads) void k_factor(Batch b, double* dbg_
 #pragma unroll
         for (int v = 0; v < 4; ++v) dt[v] = tk[64 * v + lane];
         if (K >= 0) dt = tile_update(dt, sP + 256 * (K + 1), sP + 256 * (K + 1), lane);
-        if (!factor_tile(dt, sT, sXT + 256 * (K + 1), idg + 16 * (K + 1), lane) && lane == 0) flag = 1;
+        if (!factor_tile(dt, sXT + 256 * (K + 1), idg + 16 * (K + 1), lane) && lane == 0) flag = 1;
 #pragma unroll
         for (int v = 0; v < 4; ++v) tk[64 * v + lane] = dt[v];
       }

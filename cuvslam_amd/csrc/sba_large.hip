@@ -157,7 +157,6 @@ __global__ __launch_bounds__(256) void k_potrf(Batch b, int w, int k) {
   __shared__ double sU[6 * 256];    // off-diagonal U tiles (row-major), by pair index
   __shared__ double sX[6 * 256];    // off-diagonal X tiles X_IJ (row-major), by the pair index of (J, I)
   __shared__ double sS[3 * 256];    // per-wavefront product scratch
-  __shared__ double sT[256];
   __shared__ double vec[kLB], ys[kLB], idg[kLB];
   __shared__ int flag;
   const WindowDesc W = b.win[w];
@@ -204,7 +203,7 @@ __global__ __launch_bounds__(256) void k_potrf(Batch b, int w, int k) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) dt[v] = tk[64 * v + lane];
         if (K >= 0) dt = tile_update(dt, sP + 256 * (K + 1), sP + 256 * (K + 1), lane);
-        if (!factor_tile(dt, sT, sXT + 256 * (K + 1), idg + 16 * (K + 1), lane) && lane == 0) flag = 1;
+        if (!factor_tile(dt, sXT + 256 * (K + 1), idg + 16 * (K + 1), lane) && lane == 0) flag = 1;
 #pragma unroll
         for (int v = 0; v < 4; ++v) tk[64 * v + lane] = dt[v];
       }
