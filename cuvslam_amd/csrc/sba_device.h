@@ -41,7 +41,7 @@ constexpr int kNT = 15;            // 16x16 tiles per side of the largest reduce
 constexpr int kZcLd = 240;         // leading dimension of the staged Z columns (bank-conflict free)
 constexpr int kKt = 48;            // Schur columns per tile (3 per point)
 constexpr int kFactorThreads = 512;
-constexpr int kPanel = 8;          // Cholesky panel width
+constexpr int kReduceSplit = 24;   // chunks from which a window's record reduction is split over four wavefronts
 constexpr float kFltEps = 1.1920928955078125e-7f;  // FLT_EPSILON, common/types.h:203-206
 
 struct WindowDesc {

@@ -766,6 +766,25 @@ __global__ __launch_bounds__(kBlock, 2) void k_schur(Batch b) {
   schur_dispatch<POSES_GLOBAL>(b, ch, W, lam, cur, sm);
 }
 
+// Sum over chunks c0 .. c1 of one record entry (record stride rec), eight loads in flight, in a fixed order.
+__device__ __forceinline__ float sum_records(const float* src, int64_t rec, int c0, int c1) {
+  float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  int c = c0;
+  for (; c + 8 <= c1; c += 8) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) a[k] += src[(c + k) * rec];
+  }
+  // the last ones together too: entries past the end are read from the last chunk and not added
+  if (c < c1) {
+    float x[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) x[k] = src[min(c + k, c1 - 1) * rec];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) a[k] += c + k < c1 ? x[k] : 0.f;
+  }
+  return ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+}
+
 // Sums the chunk records of each window (deterministic; no atomics). A window of many chunks: the four
 // wavefronts of a workgroup take consecutive quarters of the chunks for the same 64 record entries, each
 // summed in chunk order with eight loads in flight, and the quarters are added in a fixed order. A window of
@@ -782,36 +801,17 @@ __global__ __launch_bounds__(256) void k_reduce(Batch b) {
   const int w = lo, blk = blockIdx.x - b.red_first[w];
   const WindowDesc W = b.win[w];
   if (b.st[w].done || W.mapped) return;
-  if (W.nchunks < 64) {
+  if (W.nchunks < kReduceSplit) {
     const int64_t e = static_cast<int64_t>(blk) * 256 + threadIdx.x;
     if (e >= W.rec) return;
-    const float* src = b.part + W.part_off + e;
-    float a0 = 0.f, a1 = 0.f;
-    int c = 0;
-    for (; c + 2 <= W.nchunks; c += 2) {
-      a0 += src[c * static_cast<int64_t>(W.rec)];
-      a1 += src[(c + 1) * static_cast<int64_t>(W.rec)];
-    }
-    if (c < W.nchunks) a0 += src[c * static_cast<int64_t>(W.rec)];
-    b.sred[W.sred_off + e] = a0 + a1;
+    b.sred[W.sred_off + e] = sum_records(b.part + W.part_off + e, W.rec, 0, W.nchunks);
     return;
   }
   const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
   const int64_t e = static_cast<int64_t>(blk) * 64 + lane;
   const int64_t rec = W.rec;
   const int c0 = (W.nchunks * q) / 4, c1 = (W.nchunks * (q + 1)) / 4;
-  float s = 0.f;
-  if (e < rec) {
-    const float* src = b.part + W.part_off + e;
-    float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    int c = c0;
-    for (; c + 8 <= c1; c += 8) {
-#pragma unroll
-      for (int k = 0; k < 8; ++k) a[k] += src[(c + k) * rec];
-    }
-    for (; c < c1; ++c) a[0] += src[c * rec];
-    s = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
-  }
+  const float s = e < rec ? sum_records(b.part + W.part_off + e, rec, c0, c1) : 0.f;
   if (q > 0) sq[q - 1][lane] = s;
   __syncthreads();
   if (q == 0 && e < rec) b.sred[W.sred_off + e] = ((s + sq[0][lane]) + sq[1][lane]) + sq[2][lane];

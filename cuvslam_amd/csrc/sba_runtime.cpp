@@ -261,6 +261,7 @@ struct sba_batch {
   std::vector<void*> allocs;
   Batch dev{};
   int64_t total_obs = 0, total_pairs = 0;
+  int64_t default_chunk = 0;  // pairs per chunk chosen by default_chunk_pairs
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   double* dbg_S = nullptr;  // debug buffer of the reduced system of window 0
@@ -818,11 +819,23 @@ int check_streams(sba_handle* h, const Batch& d) {
   return SBA_OK;
 }
 
-// Pairs of work per chunk when the options leave it open: about 32 chunks per compute unit, so the hardware
-// dispatcher balances uneven windows, but at least 1024 pairs so that a chunk's record stays small against its
-// work (measured on the 512-window batch: 3000 pairs per chunk is within 2% of the best of 1000..25000).
-int64_t default_chunk_pairs(int64_t total_pairs) {
-  return std::min<int64_t>(std::max<int64_t>(1024, total_pairs / 8192), 65536);
+// Pairs of work per chunk when the options leave it open. A chunk is one workgroup that runs its tiles one after
+// another, and two workgroups fit on a compute unit, so up to 512 chunks run at once: below 1024 x 512 pairs a chunk
+// takes only its share of those, down to a single tile (a chunk never has less), as long as the records of all chunks
+// stay within kRecordBytes (`record_work`: the sum over windows of pairs x record bytes; a record is written and read
+// back once per iteration). Above, at least 1024 pairs, so that a chunk's record stays small against its work, and
+// about 32 chunks per compute unit, so that the dispatcher balances uneven windows. Measured, microseconds of the Schur
+// kernel at 1024 pairs per chunk -> at the share: 13.9k pairs 68 -> 15 (one tile per chunk), 53k pairs on 56 free key
+// frames 235 -> 41, 582k pairs 61 (the same; 512 pairs 73, 2048 pairs 96). 6.7M pairs in 128 windows: whole iterations
+// 1.29 ms at 1024, 1.28 at 1536 to 2048, 1.36 at 512 or 3072. Records of 118 KB (38 free key frames): 153k pairs 1.83 ms
+// per solve at one tile per chunk (79 MB of records), 1.75 at 384 pairs (40 MB), 2.07 at 1024; 383k pairs 2.64, 2.15 at
+// 768 (49 MB), 2.32.
+constexpr int64_t kCoarseChunkPairs = 1024;
+int64_t default_chunk_pairs(int64_t total_pairs, double record_work) {
+  constexpr int64_t kResident = 512;
+  constexpr double kRecordBytes = 40.0 * 1024 * 1024;
+  const int64_t share = std::max<int64_t>(total_pairs / kResident, static_cast<int64_t>(record_work / kRecordBytes));
+  return std::min<int64_t>(std::max<int64_t>(std::min(kCoarseChunkPairs, share), total_pairs / 8192), 65536);
 }
 
 // The launch sequence of one solve. With events, each kernel class is timed (eager mode only).
@@ -838,7 +851,7 @@ int enqueue_solve(sba_handle* h, sba_batch* b, bool timed) {
     if (timed) HIP_TRY(hipEventRecord(b->ev[1], s));
     HIP_TRY(launch_reduce(d, s));
     if (timed) HIP_TRY(hipEventRecord(b->ev[2], s));
-    HIP_TRY(launch_factor(d, nullptr, s));
+    if (b->mapped.size() < static_cast<size_t>(b->n)) HIP_TRY(launch_factor(d, nullptr, s));
     for (int w : b->mapped) HIP_TRY(launch_large_factor(d, w, 6 * b->win[w].ncf, s));
     if (timed) HIP_TRY(hipEventRecord(b->ev[3], s));
     HIP_TRY(launch_backsub(d, false, s));
@@ -1009,7 +1022,12 @@ int build_batch_impl(sba_handle* h, const sba_problem_view* problems, int32_t n,
 
   // chunks: consecutive tiles of one window, about chunk_pairs pairs of work each; each owns one record
   int64_t target = h->opt.chunk_pairs;
-  if (target <= 0) target = default_chunk_pairs(b->total_pairs);
+  if (target <= 0) {
+    double record_work = 0.0;
+    for (int w = 0; w < n; ++w) record_work += static_cast<double>(H.sorts[w].npairs) * b->win[w].rec * sizeof(float);
+    target = default_chunk_pairs(b->total_pairs, record_work);
+    b->default_chunk = target;
+  }
   const int64_t btarget = h->opt.bchunk_pairs > 0 ? h->opt.bchunk_pairs : target;
   // In a mapped window a chunk also stages at most kMaxFreePoses free key frames: its map lists them in
   // increasing order and its pairs carry their index in that list.
@@ -1138,12 +1156,12 @@ int build_batch_impl(sba_handle* h, const sba_problem_view* problems, int32_t n,
     }
   }
 
-  // record reduction work list: 64 entries per workgroup for windows of many chunks, 256 otherwise
+  // record reduction work list: 64 entries per workgroup for windows of kReduceSplit chunks or more, 256 otherwise
   pinned_vector<int32_t>& red_first = H.red_first;
   red_first.assign(n + 1, 0);
   for (int w = 0; w < n; ++w) {
     const WindowDesc& W = b->win[w];
-    const int per = W.nchunks < 64 ? 256 : 64;
+    const int per = W.nchunks < kReduceSplit ? 256 : 64;
     red_first[w + 1] = red_first[w] + (W.mapped ? 0 : (W.rec + per - 1) / per);
   }
 
@@ -1900,7 +1918,7 @@ int sba_autotune_chunks(sba_handle* h, const sba_problem_view* problems, int32_t
   if (!h || !problems || n <= 0 || !best_chunk_pairs || repeats < 1 || n_candidates < 0 || (n_candidates > 0 && !candidates))
     return fail(h, SBA_E_INVALID, "bad sba_autotune_chunks arguments");
   HIP_TRY(hipSetDevice(h->opt.device));
-  int64_t total_pairs = 0;
+  int64_t base = 0;
   {
     // the default candidates bracket the heuristic: x1/4 .. x4
     sba_batch* probe = nullptr;
@@ -1909,12 +1927,11 @@ int sba_autotune_chunks(sba_handle* h, const sba_problem_view* problems, int32_t
     const int rc = sba_batch_create(h, problems, n, &probe);
     h->opt.chunk_pairs = saved;
     if (rc != SBA_OK) return rc;
-    total_pairs = probe->total_pairs;
+    base = probe->default_chunk;
     sba_batch_destroy(h, probe);
   }
   std::vector<int32_t> cand(candidates, candidates + n_candidates);
   if (cand.empty()) {
-    const int64_t base = default_chunk_pairs(total_pairs);
     for (int64_t c : {base / 4, base / 2, base, 2 * base, 4 * base})
       cand.push_back(static_cast<int32_t>(std::max<int64_t>(256, c)));
   }
@@ -2085,14 +2102,22 @@ int sba_solve(sba_handle* h, const sba_problem_view* problem, sba_result* result
 }
 
 int sba_solve_noalloc(sba_handle* h, const sba_problem_view* problem, sba_result* result) {
-  return solve_one(h, problem, result, [h](sba_batch*, size_t bytes, char** base) -> int {
+  const MemorySource scratch = [h](sba_batch*, size_t bytes, char** base) -> int {
     if (!h->scratch) return fail(h, SBA_E_DEVICE, "the scratch array of sba_solve_noalloc is not set up");
     if (bytes > h->scratch_bytes)
       return fail(h, SBA_E_CAPACITY, "window needs " + std::to_string(bytes) + " bytes of device memory; "
                   "sba_solve_noalloc holds at most " + std::to_string(h->scratch_bytes) + " (use sba_solve)");
     *base = h->scratch;
     return SBA_OK;
-  });
+  };
+  int rc = solve_one(h, problem, result, scratch);
+  if (rc == SBA_E_CAPACITY && h->opt.chunk_pairs == 0) {
+    // small chunks trade memory for time (a record each): a window that does not fit with them may with coarse ones
+    h->opt.chunk_pairs = static_cast<int32_t>(kCoarseChunkPairs);
+    rc = solve_one(h, problem, result, scratch);
+    h->opt.chunk_pairs = 0;
+  }
+  return rc;
 }
 
 }  // extern "C"
