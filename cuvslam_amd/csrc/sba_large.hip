@@ -6,15 +6,13 @@
 //   k_gather      A = U + lambda diag(U) - sum Z Z^T in FP64 (dense, row-major lower triangle), rhs e: each
 //                 key-frame block sums its contributions from the chunk records in chunk order (a plan built
 //                 with the chunks), so the system, like the small windows' reduction, has fixed bits
-//   k_potrf / k_trsm / k_syrk   right-looking blocked Cholesky (Golub & Van Loan, Matrix Computations,
-//                 Algorithm 4.2.10) with 64 x 64 blocks: the diagonal block is factored with the 16 x 16 FP64
-//                 tile scheme of the small-window factor (matrix cores for the tile updates) and its triangular
-//                 inverse kept; the panel below it is then a product with that inverse (one block per
-//                 workgroup), the trailing update one block pair per workgroup.
-//                 The forward substitution L y = e rides along: y_k = L_kk^-1 e_k in k_potrf, e_i -= L_ik y_k
-//                 in k_trsm
-//   k_bsolve      L^T x = y by 64-row blocks with the kept inverses, in one workgroup
-//   k_lepilogue   the pose step, its max-norm and dc^T diag(U) dc, trial key frames
+//   k_lfirst / k_lstep   right-looking blocked Cholesky (Golub & Van Loan, Matrix Computations, Algorithm 4.2.10)
+//                 with 64 x 64 blocks, one launch per block column: a diagonal block is factored, with its inverse, on
+//                 the 16 x 16 FP64 tile scheme of the small-window factor; the panel below it is a product with that
+//                 inverse, formed by the workgroups of the trailing update that need it; the workgroup of the next
+//                 diagonal block goes on to factor it. The forward substitution L y = e rides along.
+//   k_bsolve      L^T x = y by 64-row blocks with the kept inverses, in one workgroup; then the pose step, its
+//                 max-norm and dc^T diag(U) dc, trial key frames
 // A non-positive pivot clears the window's chol_ok; the later kernels then return, and the LM decision raises
 // lambda (schur_complement_bundler_gpu.cpp:175-185), as for the small windows.
 #include <hip/hip_runtime.h>
@@ -35,7 +33,7 @@ constexpr int kGather = 8;     // contributions whose loads k_gather issues toge
 constexpr int kGatherWaves = 4;  // wavefronts of k_gather that share one key-frame block's contributions
 
 struct Large {
-  double* A;     // n x n, row-major; the lower triangle holds A, then L
+  double* A;     // n x n, row-major; the lower triangle holds A; L^T replaces the blocks above the diagonal
   double* rhs;   // e, then y, then x
   double* du;    // diag(U)
   double* Linv;  // per 64-row block: the inverse of its diagonal block of L (64 x 64, row-major, lower)
@@ -143,205 +141,12 @@ __global__ __launch_bounds__(64 * kGatherWaves) void k_gather(Batch b, int w) {
   }
 }
 
-// Cholesky of diagonal block k (64 x 64; rows and columns past the matrix are identity) by one workgroup of 256
-// threads, as four 16 x 16 tile columns: wavefront 0 factors the diagonal tiles (kept in LDS) one after another
-// (factor_tile), wavefronts 1..3 hold the six off-diagonal tiles U_JI (J < I, A = U^T U) in registers and apply
-// the panel step U_KI = X_KK A_KI and the trailing updates on the FP64 matrix cores; the forward-substitution
-// step y_k = L_kk^-1 e_k runs alongside. Then the block's inverse X = L_kk^-1 (for the panel GEMMs and the
-// backward solve), tile by tile: X_IJ = -X_II sum_{K=J}^{I-1} L_IK X_KJ, one tile column J per wavefront 1..3.
-__global__ __launch_bounds__(256) void k_potrf(Batch b, int w, int k) {
-  constexpr int T = kLB / 16;       // 4 tile columns
-  __shared__ double sDg[T * 256];   // diagonal tiles, row-major (U after factoring)
-  __shared__ double sXT[T * 256];   // X_KK^T per tile column (row-major)
-  __shared__ double sP[T * 256];    // panel tiles U_KI of the current tile column
-  __shared__ double sU[6 * 256];    // off-diagonal U tiles (row-major), by pair index
-  __shared__ double sX[6 * 256];    // off-diagonal X tiles X_IJ (row-major), by the pair index of (J, I)
-  __shared__ double sS[3 * 256];    // per-wavefront product scratch
-  __shared__ double vec[kLB], ys[kLB], idg[kLB];
-  __shared__ int flag;
-  const WindowDesc W = b.win[w];
-  WindowState* St = b.st + w;
-  if (St->done || !St->chol_ok) return;
-  const Large L = large_of(b, W);
-  const int n = L.n, k0 = kLB * k, kb = min(kLB, n - k0), tid = threadIdx.x;
-  const int lane = tid & 63, li = lane >> 4, lj = lane & 15;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // pair index of tile (J, I), J < I: 0 (0,1) 1 (0,2) 2 (0,3) 3 (1,2) 4 (1,3) 5 (2,3)
-  auto pair_of = [](int J, int I) { return J == 0 ? I - 1 : (J == 1 ? I + 1 : 5); };
-  // element (4v + lane/16, lane%16) of upper tile (J, I) of the symmetric block, read from the lower triangle
-  auto element = [&](int J, int I, int v) -> double {
-    const int r = 16 * J + 4 * v + li, c = 16 * I + lj;
-    if (r >= kb || c >= kb) return r == c ? 1.0 : 0.0;
-    return L.A[static_cast<int64_t>(k0 + max(r, c)) * n + k0 + min(r, c)];
-  };
-  {
-    double val[4];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) val[v] = element(wave, wave, v);  // diagonal tile `wave`
-#pragma unroll
-    for (int v = 0; v < 4; ++v) sDg[256 * wave + 64 * v + lane] = val[v];
-  }
-  if (tid < kLB) vec[tid] = tid < kb ? L.rhs[k0 + tid] : 0.0;
-  if (tid == 0) flag = 0;
+// Staged 64 x 64 operands: 16 x 16 tiles of kTs doubles with rows of kTr (one double of padding, so that the transposing
+// writes of a wavefront fall into different banks). Tile (I, M) of P, at 4 I + M, holds element [m][i] =
+// P[16 I + i][16 M + m], the operand layout of the matrix instructions (lane l reads [4q + l/16][l%16]).
+constexpr int kTr = 17, kTs = 16 * kTr;
 
-  if (wave == 0) {
-    __syncthreads();
-    for (int K = -1; K < T; ++K) {
-      if (flag) break;
-      if (K >= 0) {
-        const double* xt = sXT + 256 * K;
-        double yk = 0.0;  // y_K = X_KK e_K
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) yk += xt[16 * (4 * li + kk) + lj] * vec[16 * K + 4 * li + kk];
-        yk = sum_rows4(yk);
-        if (lane < 16) ys[16 * K + lane] = yk;
-        __syncthreads();
-      }
-      if (K + 1 < T) {
-        double* tk = sDg + 256 * (K + 1);
-        double4v dt;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) dt[v] = tk[64 * v + lane];
-        if (K >= 0) dt = tile_update(dt, sP + 256 * (K + 1), sP + 256 * (K + 1), lane);
-        if (!factor_tile(dt, sXT + 256 * (K + 1), idg + 16 * (K + 1), lane) && lane == 0) flag = 1;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) tk[64 * v + lane] = dt[v];
-      }
-      __syncthreads();
-    }
-    __syncthreads();  // the off-diagonal U tiles are published
-    __syncthreads();  // the off-diagonal X tiles are formed
-  } else {
-    // two register tiles per wavefront: pair index m = 3 s + wave - 1
-    int tJ[2], tI[2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int m = 3 * s + wave - 1;
-      tJ[s] = m < 3 ? 0 : (m < 5 ? 1 : 2);
-      tI[s] = m < 3 ? m + 1 : (m < 5 ? m - 1 : 3);
-    }
-    double4v acc[2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) acc[s][v] = element(tJ[s], tI[s], v);
-    __syncthreads();
-    for (int K = -1; K < T; ++K) {
-      if (flag) break;
-      if (K >= 0) {
-        // panel U_KI = X_KK A_KI (the B operand of chunk q is register q of the tile), e_I -= U_KI^T y_K
-        const double* xt = sXT + 256 * K;
-        double yk = 0.0;
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) yk += xt[16 * (4 * li + kk) + lj] * vec[16 * K + 4 * li + kk];
-        yk = sum_rows4(yk);
-        double yv[4];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) yv[v] = __shfl(yk, 4 * v + li);  // y_K[4v + lane/16]
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-          if (tJ[s] == K) {
-            const int I = tI[s];
-            double4v u = double4v{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int q = 0; q < 4; ++q) u = mfma64(xt[64 * q + lane], acc[s][q], u);
-            acc[s] = u;
-            double p = 0.0;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-              sP[256 * I + 64 * v + lane] = u[v];
-              p += u[v] * yv[v];
-            }
-            p = sum_rows4(p);
-            if (lane < 16) vec[16 * I + lane] -= p;
-          }
-        }
-        __syncthreads();
-        // trailing: the diagonal tiles past K + 1 (LDS), then this wavefront's tiles (J > K)
-        for (int J = K + 1 + wave; J < T; J += 3) {
-          double* tj = sDg + 256 * J;
-          double4v t;
-#pragma unroll
-          for (int v = 0; v < 4; ++v) t[v] = tj[64 * v + lane];
-          t = tile_update(t, sP + 256 * J, sP + 256 * J, lane);
-#pragma unroll
-          for (int v = 0; v < 4; ++v) tj[64 * v + lane] = t[v];
-        }
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-          if (tJ[s] > K) acc[s] = tile_update(acc[s], sP + 256 * tJ[s], sP + 256 * tI[s], lane);
-      }
-      __syncthreads();
-    }
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) sU[256 * pair_of(tJ[s], tI[s]) + 64 * v + lane] = acc[s][v];
-    __syncthreads();
-    if (flag == 0) {
-      // tile column J = wave - 1 of X: X_IJ = -X_II S, S = sum_{K=J}^{I-1} L_IK X_KJ, L_IK = U_KI^T
-      const int J = wave - 1;
-      double* S = sS + 256 * J;
-      double4v xo[3];
-#pragma unroll
-      for (int I = 1; I < T; ++I) {
-        if (I <= J) continue;
-        double4v sa = double4v{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int K = 0; K < T - 1; ++K) {
-          if (K < J || K >= I) continue;
-          const double* U = sU + 256 * pair_of(K, I);
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            // A operand L_IK[l%16][4q + l/16] = U_KI[4q + l/16][l%16]; B operand X_KJ[4q + l/16][l%16]: from
-            // X_JJ^T in LDS, or register q of the tile X_KJ formed above
-            const double xb = K == J ? sXT[256 * J + 16 * lj + 4 * q + li] : xo[K - J - 1][q];
-            sa = mfma64(U[64 * q + lane], xb, sa);
-          }
-        }
-#pragma unroll
-        for (int v = 0; v < 4; ++v) S[64 * v + lane] = sa[v];
-        wave_lds_sync();
-        // A operand X_II[l%16][4q + l/16] = X_II^T[4q + l/16][l%16]
-        double4v d = double4v{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int q = 0; q < 4; ++q) d = mfma64(-sXT[256 * I + 64 * q + lane], S[64 * q + lane], d);
-        xo[I - J - 1] = d;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) sX[256 * pair_of(J, I) + 64 * v + lane] = d[v];
-        wave_lds_sync();  // S is rewritten for the next I
-      }
-    }
-    __syncthreads();
-  }
-  __syncthreads();
-  if (flag != 0) {
-    if (tid == 0) St->chol_ok = 0;
-    return;
-  }
-  // L (lower) back to A, X = L_kk^-1 (64 x 64 row-major, zero above the diagonal) to Linv, y_k to rhs.
-  // U tile (J, I) element (r, c) is L[16 I + c][16 J + r]; X_II = (X_II^T)^T from sXT.
-  double* Xg = L.Linv + static_cast<int64_t>(k) * kLB * kLB;
-  for (int idx = tid; idx < kLB * kLB; idx += blockDim.x) {
-    const int R = idx / kLB, Cc = idx % kLB;
-    const int I = R >> 4, J = Cc >> 4, a = R & 15, c = Cc & 15;
-    double x = 0.0;
-    if (J == I) x = sXT[256 * I + 16 * c + a];
-    else if (J < I) x = sX[256 * pair_of(J, I) + 16 * a + c];
-    Xg[idx] = x;
-    if (Cc <= R && R < kb) {
-      const double l = J == I ? sDg[256 * I + 16 * c + a] : sU[256 * pair_of(J, I) + 16 * c + a];
-      L.A[static_cast<int64_t>(k0 + R) * n + k0 + Cc] = l;
-    }
-  }
-  if (tid < kb) L.rhs[k0 + tid] = ys[tid];
-}
-
-// 64 x 64 products C -= P Q^T on the FP64 matrix cores for the panel and trailing kernels below: P and Q are staged
-// in LDS as transposed 16 x 16 tiles (tile (I, M) of P at sPT + 256 (4 I + M), element [m][i] = P[16 I + i][16 M + m],
-// the operand layout of tile_update), and each of the four wavefronts owns four of the 16 output tiles (I, J)
-// = (wave, 0..3), accumulated over the four tile columns M in register tiles.
-// (256 threads: each loads its 16 entries in one batch, then stores them.)
+// 256 threads: each loads its 16 entries in one batch, then stores them.
 __device__ __forceinline__ void stage_transposed(double* sT, const double* src, int64_t ld, int rows, int cols,
                                                  int tid) {
   constexpr int kPer = kLB * kLB / 256;
@@ -354,110 +159,308 @@ __device__ __forceinline__ void stage_transposed(double* sT, const double* src, 
 #pragma unroll
   for (int it = 0; it < kPer; ++it) {
     const int idx = tid + 256 * it, r = idx / kLB, c = idx % kLB;
-    sT[256 * (4 * (r >> 4) + (c >> 4)) + 16 * (c & 15) + (r & 15)] = v[it];
+    sT[kTs * (4 * (r >> 4) + (c >> 4)) + kTr * (c & 15) + (r & 15)] = v[it];
   }
 }
 
-__device__ __forceinline__ void gemm_nt_update(double4v (&acc)[4], const double* sPT, const double* sQT, int wave,
-                                               int lane) {
+// c - P Q^T of one tile of P and one of Q, both staged as above.
+__device__ __forceinline__ double4v staged_update(double4v c, const double* p, const double* q, int at) {
+#pragma unroll
+  for (int s = 0; s < 4; ++s) c = mfma64(-p[4 * kTr * s + at], q[4 * kTr * s + at], c);
+  return c;
+}
+
+// Shared memory of factor_block, in doubles: diagonal tiles, their inverses transposed, the current panel, the
+// off-diagonal tiles of A and of X, the right-hand side.
+constexpr int kFbDg = 0, kFbXT = kFbDg + 4 * 256, kFbP = kFbXT + 4 * 256, kFbU = kFbP + 4 * 256, kFbX = kFbU + 6 * 256,
+              kFbVec = kFbX + 6 * 256, kFbY = kFbVec + kLB, kFbIdg = kFbY + kLB, kFbWords = kFbIdg + kLB;
+
+// pair index of tile (J, I), J < I < 4: 0 (0,1) 1 (0,2) 2 (0,3) 3 (1,2) 4 (1,3) 5 (2,3)
+__device__ __forceinline__ int pair_of(int J, int I) { return J == 0 ? I - 1 : (J == 1 ? I + 1 : 5); }
+
+// Cholesky A = U^T U of a 64 x 64 block by one workgroup of 256 threads, with X = U^-T and y = X e. The block's upper
+// tiles come in shared memory (sm + kFbDg, kFbU, row-major 16 x 16) and e in sm + kFbVec, with a barrier after them.
+// Wavefront 0 factors the diagonal tiles one after another (factor_tile); wavefronts 1..3 hold the six off-diagonal
+// tiles U_JI (J < I) and the six tiles X_IJ below the diagonal of the identity in registers and carry both along:
+//   panel     U_KI = X_KK A_KI, e_I -= U_KI^T y_K;   X_KJ = X_KK E_KJ;
+//   trailing  A_JI -= U_KJ^T U_KI;                   E_IJ -= U_KI^T X_KJ,
+// on the FP64 matrix cores while wavefront 0 factors the next tile, so that the block's inverse is complete when its
+// last tile is. False (in every thread) on a non-positive pivot; every thread runs the same barriers.
+// On return X is written to Xg (64 x 64 row-major, zero above the diagonal) and y to rhs.
+__device__ bool factor_block(double* sm, int* flag, double* Xg, double* rhs, int kb, int tid) {
+  constexpr int T = kLB / 16;  // 4 tile columns
+  double* sDg = sm + kFbDg;
+  double* sXT = sm + kFbXT;
+  double* sP = sm + kFbP;
+  double* sU = sm + kFbU;
+  double* sX = sm + kFbX;
+  double *vec = sm + kFbVec, *ys = sm + kFbY, *idg = sm + kFbIdg;
+  const int lane = tid & 63, li = lane >> 4, lj = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  auto forward = [&](int K) {  // y_K = X_KK e_K, lane l holds y_K[l % 16]
+    const double* xt = sXT + 256 * K;
+    double yk = 0.0;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) yk += xt[16 * (4 * li + kk) + lj] * vec[16 * K + 4 * li + kk];
+    return sum_rows4(yk);
+  };
+  if (wave == 0) {
+    for (int K = -1; K < T; ++K) {
+      if (*flag) break;
+      if (K >= 0) {
+        const double yk = forward(K);
+        if (lane < 16) ys[16 * K + lane] = yk;
+        __syncthreads();
+      }
+      if (K + 1 < T) {
+        double* tk = sDg + 256 * (K + 1);
+        double4v dt;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) dt[v] = tk[64 * v + lane];
+        if (K >= 0) dt = tile_update(dt, sP + 256 * (K + 1), sP + 256 * (K + 1), lane);
+        if (!factor_tile(dt, sXT + 256 * (K + 1), idg + 16 * (K + 1), lane) && lane == 0) *flag = 1;
+      }
+      __syncthreads();
+    }
+  } else {
+    // two register tiles of U and of X per wavefront: pair index m = 3 s + wave - 1
+    int tJ[2], tI[2];
+    double4v acc[2], inv[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int m = 3 * s + wave - 1;
+      tJ[s] = m < 3 ? 0 : (m < 5 ? 1 : 2);
+      tI[s] = m < 3 ? m + 1 : (m < 5 ? m - 1 : 3);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) acc[s][v] = sU[256 * m + 64 * v + lane];
+      inv[s] = double4v{0.0, 0.0, 0.0, 0.0};
+    }
+    for (int K = -1; K < T; ++K) {
+      if (*flag) break;
+      if (K >= 0) {
+        const double* xt = sXT + 256 * K;
+        const double yk = forward(K);
+        double yv[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) yv[v] = __shfl(yk, 4 * v + li);  // y_K[4v + lane/16]
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          if (tJ[s] == K || tI[s] == K) {
+            // X_KK times a tile: the B operand of chunk q is register q of the tile
+            const double4v in = tJ[s] == K ? acc[s] : inv[s];
+            double4v u = double4v{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) u = mfma64(xt[64 * q + lane], in[q], u);
+            double* dst = tJ[s] == K ? sP + 256 * tI[s] : sX + 256 * pair_of(tJ[s], K);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) dst[64 * v + lane] = u[v];
+            if (tJ[s] == K) {
+              double p = 0.0;
+#pragma unroll
+              for (int v = 0; v < 4; ++v) p += u[v] * yv[v];
+              p = sum_rows4(p);
+              if (lane < 16) vec[16 * tI[s] + lane] -= p;
+            }
+          }
+        }
+        __syncthreads();
+        // trailing: the diagonal tiles past K + 1 (LDS), then this wavefront's tiles
+        for (int J = K + 1 + wave; J < T; J += 3) {
+          double* tj = sDg + 256 * J;
+          double4v t;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) t[v] = tj[64 * v + lane];
+          t = tile_update(t, sP + 256 * J, sP + 256 * J, lane);
+#pragma unroll
+          for (int v = 0; v < 4; ++v) tj[64 * v + lane] = t[v];
+        }
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          if (tJ[s] > K) {
+            acc[s] = tile_update(acc[s], sP + 256 * tJ[s], sP + 256 * tI[s], lane);
+          } else if (tI[s] > K) {
+            // B operand X_KJ[4q + l/16][l%16]: X_KK from its transpose, the others row-major
+            const double* U = sP + 256 * tI[s];
+            const double* X = tJ[s] == K ? xt + 16 * lj + li : sX + 256 * pair_of(tJ[s], K) + lane;
+            const int step = tJ[s] == K ? 4 : 64;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) inv[s] = mfma64(-U[64 * q + lane], X[step * q], inv[s]);
+          }
+        }
+      }
+      __syncthreads();
+    }
+  }
+  if (*flag) return false;
+  for (int idx = tid; idx < kLB * kLB; idx += 256) {
+    const int R = idx / kLB, Cc = idx % kLB;
+    const int I = R >> 4, J = Cc >> 4, a = R & 15, c = Cc & 15;
+    double x = 0.0;
+    if (J == I) x = sXT[256 * I + 16 * c + a];
+    else if (J < I) x = sX[256 * pair_of(J, I) + 16 * a + c];
+    Xg[idx] = x;
+  }
+  if (tid < kb) rhs[tid] = ys[tid];
+  return true;
+}
+
+// The first diagonal block: read, factored, its inverse and y_0 written.
+__global__ __launch_bounds__(256) void k_lfirst(Batch b, int w) {
+  __shared__ double sm[kFbWords];
+  __shared__ int flag;
+  const WindowDesc W = b.win[w];
+  WindowState* St = b.st + w;
+  if (St->done || !St->chol_ok) return;
+  const Large L = large_of(b, W);
+  const int n = L.n, kb = min(kLB, n), tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  // upper tiles (wave, I), read from the lower triangle; identity past the matrix
+  for (int I = wave; I < 4; ++I) {
+    double* dst = I == wave ? sm + kFbDg + 256 * I : sm + kFbU + 256 * pair_of(wave, I);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int r = 16 * wave + 4 * v + (lane >> 4), c = 16 * I + (lane & 15);
+      dst[64 * v + lane] = r < kb && c < kb ? L.A[static_cast<int64_t>(max(r, c)) * n + min(r, c)] : (r == c ? 1.0 : 0.0);
+    }
+  }
+  if (tid < kLB) sm[kFbVec + tid] = tid < kb ? L.rhs[tid] : 0.0;
+  if (tid == 0) flag = 0;
+  __syncthreads();
+  if (!factor_block(sm, &flag, L.Linv, L.rhs, kb, tid) && tid == 0) St->chol_ok = 0;
+}
+
+// Step k of the right-looking factorization, one workgroup per block (i, j), k < j <= i, of what is left. Block k's
+// inverse X is known, so each workgroup forms the panel blocks it needs itself, L_ik = A_ik X^T and L_jk = A_jk X^T, and
+// subtracts L_ik L_jk^T from A_ij: recomputing a panel block costs a 64-wide product (10 of 16 tiles, X being
+// triangular), less than the launch that a separate panel kernel would cost. The workgroup of (i, i) also keeps L_ik,
+// transposed, in the unused upper triangle (block (k, i); the lower A_ik is still read by others) for the backward
+// solve, and takes e_i -= L_ik y_k. The first workgroup, block (k + 1, k + 1), goes on to factor its block
+// (factor_block), so the next step starts with its inverse: one launch per block column, bound by that workgroup's serial
+// chain. Order 1194: 24 us per block column, against 45 us with separate diagonal, panel and trailing launches (24 + 11
+// + 10); order 336: 23.5 against 43.
+__global__ __launch_bounds__(256) void k_lstep(Batch b, int w, int k) {
+  __shared__ double sm[3 * 16 * kTs];
+  __shared__ double sy[kLB], sred[4 * kLB];
+  __shared__ int flag;
+  static_assert(kFbWords <= 3 * 16 * kTs, "factor_block reuses the staging memory");
+  const WindowDesc W = b.win[w];
+  WindowState* St = b.st + w;
+  if (St->done || !St->chol_ok) return;
+  const Large L = large_of(b, W);
+  const int n = L.n, k0 = kLB * k, tid = threadIdx.x;  // block k is a full one: blocks follow it
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int at = kTr * (lane >> 4) + (lane & 15);
+  int ii = 0, jj = blockIdx.x;  // 0 <= jj <= ii, row by row
+  while (jj > ii) jj -= ++ii;
+  const bool diag = ii == jj;
+  const int i0 = kLB * (k + 1 + ii), j0 = kLB * (k + 1 + jj);
+  const int ib = min(kLB, n - i0), jb = min(kLB, n - j0);
+  double* sX = sm;                // X
+  double* sA = sm + 16 * kTs;     // A_ik, then L_ik
+  double* sB = diag ? sA : sm + 32 * kTs;  // A_jk, then L_jk
+  if (tid == 0) flag = 0;
+  stage_transposed(sX, L.Linv + static_cast<int64_t>(k) * kLB * kLB, kLB, kLB, kLB, tid);
+  stage_transposed(sA, L.A + static_cast<int64_t>(i0) * n + k0, n, ib, kLB, tid);
+  if (!diag) stage_transposed(sB, L.A + static_cast<int64_t>(j0) * n + k0, n, jb, kLB, tid);
+  if (tid < kLB) sy[tid] = L.rhs[k0 + tid];
+  // this wavefront's tiles (wave, J) of A_ij, element (4 v + lane / 16, lane % 16) in register v
+  double4v acc[4];
+#pragma unroll
+  for (int J = 0; J < 4; ++J)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      // a diagonal block: symmetric, read from its lower triangle, identity past the matrix
+      const int r0 = 16 * wave + 4 * v + (lane >> 4), c0 = 16 * J + (lane & 15);
+      const int r = diag ? max(r0, c0) : r0, c = diag ? min(r0, c0) : c0;
+      acc[J][v] = (r0 < ib && c0 < jb) ? L.A[static_cast<int64_t>(i0 + r) * n + j0 + c] : (diag && r0 == c0 ? 1.0 : 0.0);
+    }
+  __syncthreads();
+  // The transposed panel tiles (L_ik^T)(J, wave) = sum_M X(J, M) A_ik(wave, M)^T come out in the staged layout; they
+  // replace the tiles (wave, J) of A_ik, which only this wavefront reads.
+  auto panel = [&](double* sS) {
+    double4v p[4];
+#pragma unroll
+    for (int J = 0; J < 4; ++J) {
+      p[J] = double4v{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int M = 0; M <= J; ++M)
+        p[J] = staged_update(p[J], sX + kTs * (4 * J + M), sS + kTs * (4 * wave + M), at);
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int J = 0; J < 4; ++J)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        p[J][v] = -p[J][v];
+        sS[kTs * (4 * wave + J) + 4 * kTr * v + at] = p[J][v];
+      }
+    return [=](int J, int v) { return p[J][v]; };
+  };
+  const auto pi = panel(sA);
+  if (!diag) {
+    panel(sB);
+  } else {
+#pragma unroll
+    for (int J = 0; J < 4; ++J)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int c = 16 * J + 4 * v + (lane >> 4), r = 16 * wave + (lane & 15);
+        if (r < ib) L.A[static_cast<int64_t>(k0 + c) * n + i0 + r] = pi(J, v);
+      }
+  }
+  __syncthreads();
 #pragma unroll
   for (int J = 0; J < 4; ++J)
 #pragma unroll
     for (int M = 0; M < 4; ++M)
-      acc[J] = tile_update(acc[J], sPT + 256 * (4 * wave + M), sQT + 256 * (4 * J + M), lane);
-}
-
-// Panel below diagonal block k: L_ik = A_ik L_kk^-T = A_ik X^T with the kept inverse X, one block row per
-// workgroup, on the matrix cores; then the block row's forward-substitution update e_i -= L_ik y_k.
-__global__ __launch_bounds__(256) void k_trsm(Batch b, int w, int k) {
-  __shared__ double sAT[16 * 256];
-  __shared__ double sXT[16 * 256];
-  __shared__ double sy[kLB];
-  const WindowDesc W = b.win[w];
-  WindowState* St = b.st + w;
-  if (St->done || !St->chol_ok) return;
-  const Large L = large_of(b, W);
-  const int n = L.n, k0 = kLB * k, kb = min(kLB, n - k0), tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int i0 = kLB * (k + 1 + blockIdx.x), ib = min(kLB, n - i0);
-  const double* X = L.Linv + static_cast<int64_t>(k) * kLB * kLB;
-  stage_transposed(sAT, L.A + static_cast<int64_t>(i0) * n + k0, n, ib, kb, tid);
-  stage_transposed(sXT, X, kLB, kLB, kLB, tid);
-  if (tid < kLB) sy[tid] = tid < kb ? L.rhs[k0 + tid] : 0.0;
-  __syncthreads();
-  double4v acc[4];
-#pragma unroll
-  for (int J = 0; J < 4; ++J) acc[J] = double4v{0.0, 0.0, 0.0, 0.0};
-  gemm_nt_update(acc, sAT, sXT, wave, lane);  // -(A X^T) for the tiles (wave, J)
-  __syncthreads();  // every wavefront has read sAT before it is overwritten with L_ik (row-major)
-  double* sL = sAT;
-#pragma unroll
-  for (int J = 0; J < 4; ++J)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int r = 16 * wave + 4 * v + (lane >> 4), c = 16 * J + (lane & 15);
-      const double val = (r < ib && c < kb) ? -acc[J][v] : 0.0;
-      sL[r * kLB + c] = val;
-      if (r < ib && c < kb) L.A[static_cast<int64_t>(i0 + r) * n + k0 + c] = val;
-    }
-  __syncthreads();
-  if (tid < ib) {
+      acc[J] = staged_update(acc[J], sA + kTs * (4 * wave + M), sB + kTs * (4 * J + M), at);
+  double e = 0.0;
+  if (diag) {  // e_i -= L_ik y_k: wavefront g sums columns 16 g .. 16 g + 15 of row `lane`
     double s = 0.0;
-    for (int m = 0; m < kb; ++m) s += sL[tid * kLB + m] * sy[m];
-    L.rhs[i0 + tid] -= s;
-  }
-}
-
-// Trailing update after block k: A_ij -= L_ik L_jk^T for k < j <= i, one block pair per workgroup, on the matrix
-// cores (the lower triangle of a diagonal block).
-__global__ __launch_bounds__(256) void k_syrk(Batch b, int w, int k) {
-  __shared__ double sAT[16 * 256];
-  __shared__ double sBT[16 * 256];
-  const WindowDesc W = b.win[w];
-  WindowState* St = b.st + w;
-  if (St->done || !St->chol_ok) return;
-  const Large L = large_of(b, W);
-  const int n = L.n, k0 = kLB * k, kb = min(kLB, n - k0), tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  int ii = 0, t = blockIdx.x;
-  while (t > ii) {
-    t -= ii + 1;
-    ++ii;
-  }
-  const int jj = t;  // 0 <= jj <= ii
-  const int i0 = kLB * (k + 1 + ii), j0 = kLB * (k + 1 + jj);
-  const int ib = min(kLB, n - i0), jb = min(kLB, n - j0);
-  stage_transposed(sAT, L.A + static_cast<int64_t>(i0) * n + k0, n, ib, kb, tid);
-  stage_transposed(sBT, L.A + static_cast<int64_t>(j0) * n + k0, n, jb, kb, tid);
-  // this wavefront's output tiles (wave, J), element (4 v + lane / 16, lane % 16) in register v
-  double4v acc[4];
 #pragma unroll
-  for (int J = 0; J < 4; ++J)
+    for (int m = 0; m < 16; ++m) s += sA[kTs * (4 * (lane >> 4) + wave) + kTr * m + (lane & 15)] * sy[16 * wave + m];
+    sred[kLB * wave + lane] = s;
+    __syncthreads();
+    if (tid < ib) e = L.rhs[i0 + tid] - ((sred[tid] + sred[kLB + tid]) + (sred[2 * kLB + tid] + sred[3 * kLB + tid]));
+  }
+  if (blockIdx.x != 0) {
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int r = 16 * wave + 4 * v + (lane >> 4), c = 16 * J + (lane & 15);
-      acc[J][v] = (r < ib && c < jb) ? L.A[static_cast<int64_t>(i0 + r) * n + j0 + c] : 0.0;
-    }
+    for (int J = 0; J < 4; ++J)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int r = 16 * wave + 4 * v + (lane >> 4), c = 16 * J + (lane & 15);
+        if (r < ib && c < jb && (!diag || c <= r)) L.A[static_cast<int64_t>(i0 + r) * n + j0 + c] = acc[J][v];
+      }
+    if (diag && tid < ib) L.rhs[i0 + tid] = e;
+    return;
+  }
+  // block (k + 1, k + 1): its upper tiles and right-hand side to factor_block (the barrier above ended the reads of sm)
+#pragma unroll
+  for (int J = 0; J < 4; ++J) {
+    if (J < wave) continue;
+    double* dst = J == wave ? sm + kFbDg + 256 * J : sm + kFbU + 256 * pair_of(wave, J);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) dst[64 * v + lane] = acc[J][v];
+  }
+  if (tid < kLB) sm[kFbVec + tid] = e;
   __syncthreads();
-  gemm_nt_update(acc, sAT, sBT, wave, lane);
-#pragma unroll
-  for (int J = 0; J < 4; ++J)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int r = 16 * wave + 4 * v + (lane >> 4), c = 16 * J + (lane & 15);
-      if (r < ib && c < jb && (ii != jj || c <= r)) L.A[static_cast<int64_t>(i0 + r) * n + j0 + c] = acc[J][v];
-    }
+  if (!factor_block(sm, &flag, L.Linv + static_cast<int64_t>(k + 1) * kLB * kLB, L.rhs + i0, ib, tid) && tid == 0)
+    St->chol_ok = 0;
 }
 
-// Backward substitution L^T x = y in one workgroup of 1024 threads, 64-row blocks from the last: for block bk,
-// r = y_bk - sum_{i past the block} L[i][block bk]^T x_i (16 groups of 64 threads, each group one row at a time
-// with its 64 lanes on the block's 64 contiguous columns), then x_bk = X_bk^T r with the kept inverse. x stays
-// in the dynamic shared memory (n doubles) and goes to rhs at the end.
+// Backward substitution L^T x = y in one workgroup of 1024 threads, 64-row blocks from the last, then the pose step, its
+// max-norm, dc^T diag(U) dc and the trial key frames. For block bk, r = y_bk - sum_{i past the block} L[i][block bk]^T
+// x_i: the rows of L^T lie in the upper triangle (k_lstep), so each of the 16 wavefronts takes four rows with its lanes
+// along them, 16 loads of 16 bytes of a lane in flight, and adds its lanes; then x_bk = X_bk^T r with the kept
+// inverse, whose loads do not wait for r. x stays in the dynamic shared memory (n doubles). The latency of one
+// workgroup's loads bounds it: order 1194, 5.7 MB, 101 us, the epilogue (8 us as a launch of its own) included; 110 us
+// with the rows gathered down the columns of L, 141 with 8-byte loads along the rows.
 __global__ __launch_bounds__(1024) void k_bsolve(Batch b, int w) {
-  constexpr int kG = 16;                        // row groups
-  extern __shared__ double sx[];                 // y, overwritten by x block by block
+  constexpr int kG = 16;             // wavefronts
+  constexpr int kR = kLB / kG;       // rows of a block per wavefront
+  extern __shared__ double sx[];     // y, overwritten by x block by block
   __shared__ double part[kG * kLB];
   __shared__ double sr[kLB];
+  __shared__ double red[2 * kG];
   const WindowDesc W = b.win[w];
   WindowState* St = b.st + w;
   if (St->done || !St->chol_ok) return;
@@ -468,35 +471,44 @@ __global__ __launch_bounds__(1024) void k_bsolve(Batch b, int w) {
   __syncthreads();
   for (int bk = nb - 1; bk >= 0; --bk) {
     const int b0 = kLB * bk, bb = min(kLB, n - b0);
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;  // four rows in flight per thread
-    if (c < bb) {
-      const double* col = L.A + b0 + c;
-      int i = b0 + kLB + g;
-      for (; i + 3 * kG < n; i += 4 * kG) {
-        s0 += col[static_cast<int64_t>(i) * n] * sx[i];
-        s1 += col[static_cast<int64_t>(i + kG) * n] * sx[i + kG];
-        s2 += col[static_cast<int64_t>(i + 2 * kG) * n] * sx[i + 2 * kG];
-        s3 += col[static_cast<int64_t>(i + 3 * kG) * n] * sx[i + 3 * kG];
-      }
-      for (; i < n; i += kG) s0 += col[static_cast<int64_t>(i) * n] * sx[i];
-    }
-    part[g * kLB + c] = (s0 + s1) + (s2 + s3);
-    __syncthreads();
-    if (tid < kLB) {
-      double r = 0.0;
-      if (c < bb) {
-        r = sx[b0 + c];
+    // rows kR g .. kR g + kR - 1 of X_bk (zero above the diagonal), column c
+    const double* X = L.Linv + static_cast<int64_t>(bk) * kLB * kLB + kR * g * kLB + c;
+    double xv[kR];
 #pragma unroll
-        for (int q = 0; q < kG; ++q) r -= part[q * kLB + c];
+    for (int r = 0; r < kR; ++r) xv[r] = X[r * kLB];
+    double s[kR] = {};
+    // rows past the matrix (only in the last block, which has nothing past it) are not reached
+    const double2* row = reinterpret_cast<const double2*>(L.A + static_cast<int64_t>(b0 + kR * g) * n);
+    const int h = n / 2;  // n is even (6 per key frame), so rows and column pairs are 16-byte aligned
+    for (int i = (b0 + kLB) / 2 + c; i < h; i += 4 * 64) {
+      double2 v[4][kR];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int r = 0; r < kR; ++r) v[u][r] = row[static_cast<int64_t>(r) * h + min(i + 64 * u, h - 1)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int q = i + 64 * u;
+        const double x0 = q < h ? sx[2 * q] : 0.0, x1 = q < h ? sx[2 * q + 1] : 0.0;
+#pragma unroll
+        for (int r = 0; r < kR; ++r) s[r] += v[u][r].x * x0 + v[u][r].y * x1;
       }
-      sr[c] = r;
+    }
+    // the four rows' sums over the lanes: lanes exchange two rows, then one, so that each 16 lanes end with one row
+    static_assert(kR == 4, "the exchange below covers four rows");
+    const bool hi = c & 32, odd = c & 16;
+    const double t0 = hi ? s[2] : s[0], t1 = hi ? s[3] : s[1];
+    const double q0 = t0 + __shfl_xor(hi ? s[0] : s[2], 32), q1 = t1 + __shfl_xor(hi ? s[1] : s[3], 32);
+    const double sum = sum_row16_dpp((odd ? q1 : q0) + __shfl_xor(odd ? q0 : q1, 16));
+    if ((c & 15) == 0) {
+      const int r = kR * g + (c >> 4);
+      sr[r] = r < bb ? sx[b0 + r] - sum : 0.0;
     }
     __syncthreads();
-    // x_c = sum_{m >= c} X[m][c] r_m, the sum split over the 16 groups
-    const double* X = L.Linv + static_cast<int64_t>(bk) * kLB * kLB;
+    // x_c = sum_{m >= c} X[m][c] r_m, four rows per wavefront, added in wavefront order
     double xs = 0.0;
-    if (c < bb)
-      for (int m = c + g; m < bb; m += kG) xs += X[m * kLB + c] * sr[m];
+#pragma unroll
+    for (int r = 0; r < kR; ++r) xs += xv[r] * sr[kR * g + r];
     part[g * kLB + c] = xs;
     __syncthreads();
     if (tid < bb) {
@@ -507,21 +519,10 @@ __global__ __launch_bounds__(1024) void k_bsolve(Batch b, int w) {
     }
     __syncthreads();
   }
-  for (int i = tid; i < n; i += blockDim.x) L.rhs[i] = sx[i];
-}
-
-// The pose step, max |dc|, dc^T diag(U) dc and the trial key frames of window w.
-__global__ __launch_bounds__(256) void k_lepilogue(Batch b, int w) {
-  __shared__ double red[8];
-  const WindowDesc W = b.win[w];
-  WindowState* St = b.st + w;
-  if (St->done || !St->chol_ok) return;
-  const Large L = large_of(b, W);
-  const int n = L.n, tid = threadIdx.x, lane = tid & 63;
   double sc = 0.0;
   float mx = 0.f;
   for (int i = tid; i < n; i += blockDim.x) {
-    const double x = L.rhs[i];
+    const double x = sx[i];
     b.dc[W.dc_off + i] = static_cast<float>(x);
     b.dc64[W.dc_off + i] = x;
     sc += x * x * L.du[i];
@@ -532,40 +533,39 @@ __global__ __launch_bounds__(256) void k_lepilogue(Batch b, int w) {
     sc += __shfl_xor(sc, o);
     mx = fmaxf(mx, __shfl_xor(mx, o));
   }
-  if (lane == 0) {
-    red[tid >> 6] = sc;
-    red[4 + (tid >> 6)] = static_cast<double>(mx);
+  if (c == 0) {
+    red[g] = sc;
+    red[kG + g] = static_cast<double>(mx);
   }
   __syncthreads();
   if (tid == 0) {
-    St->scal_pose = red[0] + red[1] + red[2] + red[3];
-    St->maxdc = static_cast<float>(fmax(fmax(red[4], red[5]), fmax(red[6], red[7])));
+    double t = 0.0, m = 0.0;
+    for (int q = 0; q < kG; ++q) {
+      t += red[q];
+      m = fmax(m, red[kG + q]);
+    }
+    St->scal_pose = t;
+    St->maxdc = static_cast<float>(m);
   }
-  write_trial_poses(b, W, St->cur, L.rhs, tid, blockDim.x);
+  write_trial_poses(b, W, St->cur, sx, tid, blockDim.x);
 }
 
 namespace sba_dev {
 
-// The factor and solve of window w (n = 6 free key frames): gather, blocked Cholesky, triangular solves,
-// epilogue. 3 nb launches for nb 64-row blocks.
+// The factor and solve of window w (n = 6 free key frames): gather, blocked Cholesky, backward solve and epilogue. One
+// launch per 64-row block and two besides.
 hipError_t launch_large_factor(const Batch& b, int w, int n, hipStream_t s) {
   const int nb = (n + kLB - 1) / kLB, ncf = n / 6;
   hipLaunchKernelGGL(k_gather, dim3(ncf * (ncf + 1) / 2), dim3(64 * kGatherWaves), 0, s, b, w);
+  hipLaunchKernelGGL(k_lfirst, dim3(1), dim3(256), 0, s, b, w);
   hipError_t e = hipGetLastError();
-  for (int k = 0; k < nb && e == hipSuccess; ++k) {
-    hipLaunchKernelGGL(k_potrf, dim3(1), dim3(256), 0, s, b, w, k);
+  for (int k = 0; k + 1 < nb && e == hipSuccess; ++k) {
     const int m = nb - k - 1;
-    if (m > 0) {
-      hipLaunchKernelGGL(k_trsm, dim3(m), dim3(256), 0, s, b, w, k);
-      hipLaunchKernelGGL(k_syrk, dim3(m * (m + 1) / 2), dim3(256), 0, s, b, w, k);
-    }
+    hipLaunchKernelGGL(k_lstep, dim3(m * (m + 1) / 2), dim3(256), 0, s, b, w, k);
     e = hipGetLastError();
   }
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_bsolve, dim3(1), dim3(1024), sizeof(double) * n, s, b, w);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_lepilogue, dim3(1), dim3(256), 0, s, b, w);
   return hipGetLastError();
 }
 
