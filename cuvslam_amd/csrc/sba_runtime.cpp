@@ -28,6 +28,7 @@
 #include <rocprofiler-sdk-roctx/roctx.h>
 
 #include "../../include/cuvslam_sba.h"
+#include "sba_adjoint.h"
 #include "sba_device.h"
 
 namespace sba_dev {
@@ -35,15 +36,12 @@ hipError_t launch_reset(const Batch& b, hipStream_t s);
 hipError_t launch_schur(const Batch& b, hipStream_t s);
 hipError_t launch_reduce(const Batch& b, hipStream_t s);
 hipError_t launch_factor(const Batch& b, double* dbg_S, hipStream_t s, double* store_L = nullptr);
-hipError_t launch_adj_obs(const Batch& b, int mode, const double* spts, const double* sposes, const double* v, double* y,
-                          double* ec, const double* zc, double* dxy, double* dinfo, const int32_t* orig, int32_t* done,
-                          hipStream_t s);
 hipError_t launch_adj_state(const Batch& b, double* spts, double* sposes, const double* a, int op, hipStream_t s);
-hipError_t launch_adj_linv(const double* Lst, int n, double* Linv, hipStream_t s);
-hipError_t launch_adj_chol(const double* Linv, int n, const double* ec, double* zc, const int32_t* done, hipStream_t s);
-hipError_t launch_adj_vec(const Batch& b, double* x, double* r, double* z, double* p, double* y, double* ec, double* zc,
-                          double* acc, double* g, double* sc, int32_t* done, double tol, int nx, int n6, int op,
-                          hipStream_t s);
+hipError_t launch_adj_assemble(const Batch& b, const AdjData& A, bool hess, hipStream_t s);
+hipError_t launch_adj_start(const Batch& b, const AdjData& A, hipStream_t s);
+hipError_t launch_adj_iteration(const Batch& b, AdjData A, int it, hipStream_t s);
+hipError_t launch_adj_obs_grad(const Batch& b, const AdjData& A, const int32_t* orig, hipStream_t s);
+hipError_t launch_adj_inverse(const double* Lst, int n, double* Linv, double* sinv, hipStream_t s);
 hipError_t launch_backsub(const Batch& b, bool initial, hipStream_t s);
 hipError_t launch_large_factor(const Batch& b, int w, int n, hipStream_t s);
 hipError_t launch_winsorize_select(const Batch& b, int w, int np, int kf, double* err, int32_t* pt_of,
@@ -261,6 +259,7 @@ struct sba_batch {
   std::vector<void*> allocs;
   Batch dev{};
   int64_t total_obs = 0, total_pairs = 0;
+  int pairs0 = 0, btiles0 = 0;  // pairs and back-substitution tiles of window 0 (they come first)
   int64_t default_chunk = 0;  // pairs per chunk chosen by default_chunk_pairs
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
@@ -1020,6 +1019,8 @@ int build_batch_impl(sba_handle* h, const sba_problem_view* problems, int32_t n,
   b->total_obs = static_cast<int64_t>(H.obs_xy.size());
   b->total_pairs = static_cast<int64_t>(H.pair_pose.size());
 
+  b->pairs0 = H.sorts[0].npairs;
+  b->btiles0 = static_cast<int>(H.wbtiles[0].size());
   // chunks: consecutive tiles of one window, about chunk_pairs pairs of work each; each owns one record
   int64_t target = h->opt.chunk_pairs;
   if (target <= 0) {
@@ -1717,50 +1718,61 @@ int sba_debug_copy(sba_handle* h, int64_t bytes, int32_t repeats, float* ms) {
 namespace {
 
 // Workspace of the implicit-differentiation path of window 0 (FP64, one allocation).
-struct AdjWork {
-  int n6, nx, no;
-  double *x, *r, *z, *p, *y, *ec, *zc, *acc, *gd, *sc, *Lst, *Linv, *dxy, *dinfo, *spts, *sposes;
-  int32_t* done;
-};
-
-int adj_workspace(sba_handle* h, sba_batch* b, AdjWork& A) {
+int adj_workspace(sba_handle* h, sba_batch* b, AdjData& A) {
   const WindowDesc& W = b->win[0];
-  A.n6 = 6 * W.ncf;
-  A.nx = A.n6 + 3 * W.npf;
-  A.no = W.no;
-  const int64_t npk = static_cast<int64_t>(A.n6) * (A.n6 + 1) / 2;
-  // x r z p y ec zc acc g (nx each), sc (8), done (2), factor (npk + n6), its inverse (n6 x n6), dxy (2 no),
-  // dinfo (3 no), FP64 points (3 np) and key frames (12 nc)
-  const size_t nx = static_cast<size_t>(A.nx);
-  const size_t nd = 9 * nx + 8 + 2 + static_cast<size_t>(npk + A.n6) + static_cast<size_t>(A.n6) * A.n6 +
-                    5 * static_cast<size_t>(A.no) + 3 * static_cast<size_t>(W.np) + 12 * static_cast<size_t>(W.nc);
+  const size_t n6 = 6 * static_cast<size_t>(W.ncf), npf = W.npf, nx = n6 + 3 * npf, np = W.np, nc = W.nc, no = W.no;
+  const size_t pairs = b->pairs0, npk = n6 * (n6 + 1) / 2;
+  A.n6 = static_cast<int>(n6);
+  A.nx = static_cast<int>(nx);
+  A.npf = W.npf;
+  A.pairs = b->pairs0;
+  A.obs = W.no;
+  A.tiles = b->btiles0;
+  A.slots = std::max(1, std::min(kAdjSlots, A.tiles));
+  size_t total = 0;
+  char* base = reinterpret_cast<char*>(b->adj);
+  auto take = [&](double*& p, size_t count) {
+    p = reinterpret_cast<double*>(base + total);
+    total += (std::max<size_t>(count, 1) * sizeof(double) + 255) & ~size_t(255);
+  };
+  auto lay_out = [&] {
+    total = 0;
+    for (double** v : {&A.x, &A.r, &A.z, &A.p, &A.y, &A.gd}) take(*v, nx);
+    take(A.spts, 3 * np);
+    take(A.sposes, 12 * nc);
+    take(A.pc, 2 * 6 * kMaxFreePoses);
+    take(A.zc, n6);
+    take(A.jac, 21 * no);
+    take(A.wh, 18 * pairs);
+    take(A.wg, 18 * pairs);
+    take(A.vh, 6 * npf);
+    take(A.uh, 6 * n6);
+    take(A.part, static_cast<size_t>(A.slots) * 27 * W.ncf);
+    take(A.part2, static_cast<size_t>(A.slots) * n6);
+    for (double** v : {&A.s_rz, &A.s_py, &A.s_rr}) take(*v, A.slots);
+    take(A.sc, 8);
+    take(A.lst, npk + n6);
+    take(A.linv, n6 * n6);
+    take(A.sinv, n6 * n6);
+    take(A.dxy, 2 * no);
+    take(A.dinfo, 3 * no);
+    double* done = nullptr;
+    take(done, 1);
+    A.done = reinterpret_cast<int32_t*>(done);
+  };
+  lay_out();
   if (!b->adj) {
-    HIP_TRY(hipMalloc(&b->adj, nd * sizeof(double)));
+    HIP_TRY(hipMalloc(&b->adj, total));
     b->allocs.push_back(b->adj);
+    base = reinterpret_cast<char*>(b->adj);
+    lay_out();
   }
-  A.x = b->adj;
-  A.r = A.x + nx;
-  A.z = A.r + nx;
-  A.p = A.z + nx;
-  A.y = A.p + nx;
-  A.ec = A.y + nx;
-  A.zc = A.ec + nx;
-  A.acc = A.zc + nx;
-  A.gd = A.acc + nx;
-  A.sc = A.gd + nx;
-  A.done = reinterpret_cast<int32_t*>(A.sc + 8);
-  A.Lst = A.sc + 10;
-  A.Linv = A.Lst + npk + A.n6;
-  A.dxy = A.Linv + static_cast<size_t>(A.n6) * A.n6;
-  A.dinfo = A.dxy + 2 * static_cast<size_t>(A.no);
-  A.spts = A.dinfo + 3 * static_cast<size_t>(A.no);
-  A.sposes = A.spts + 3 * static_cast<size_t>(W.np);
   return SBA_OK;
 }
 
 // Factors the Gauss-Newton system of the solution of window 0 (lambda = 0) once and copies its state to FP64.
 // The batch's LM state is left as it was.
-int adj_prepare(sba_handle* h, sba_batch* b, AdjWork& A) {
+int adj_prepare(sba_handle* h, sba_batch* b, AdjData& A) {
   if (b->win[0].mapped)
     return fail(h, SBA_E_CAPACITY, "implicit differentiation supports windows of at most 40 free key frames");
   int rc = adj_workspace(h, b, A);
@@ -1784,8 +1796,8 @@ int adj_prepare(sba_handle* h, sba_batch* b, AdjWork& A) {
   }
   WindowState chk{};
   if (launch_adj_state(d, A.spts, A.sposes, nullptr, 0, s) != hipSuccess || launch_schur(d, s) != hipSuccess ||
-      launch_reduce(d, s) != hipSuccess || launch_factor(d, nullptr, s, A.Lst) != hipSuccess ||
-      launch_adj_linv(A.Lst, A.n6, A.Linv, s) != hipSuccess) {
+      launch_reduce(d, s) != hipSuccess || launch_factor(d, nullptr, s, A.lst) != hipSuccess ||
+      launch_adj_inverse(A.lst, A.n6, A.linv, A.sinv, s) != hipSuccess) {
     rc = fail(h, SBA_E_DEVICE, "adjoint factor launch failed");
   } else if (hipMemcpyAsync(&chk, d.st, sizeof(chk), hipMemcpyDeviceToHost, s) != hipSuccess ||
              hipStreamSynchronize(s) != hipSuccess) {
@@ -1800,61 +1812,23 @@ int adj_prepare(sba_handle* h, sba_batch* b, AdjWork& A) {
   return rc;
 }
 
-// x = H^-1 gd by preconditioned conjugate gradients; the iteration count lands in sc[3]. The iterations are
-// enqueued in blocks of kCgBlock and the host reads the device's convergence flag after each block, so a solve
-// that converges early does not enqueue the remaining iterations (which would only idle on the flag).
+// x = H^-1 gd by preconditioned conjugate gradients on the assembled blocks; the iteration count lands in sc[2]. The
+// iterations are enqueued in blocks of kCgBlock and the host reads the device's convergence flag after each block, so a
+// solve that converges early does not enqueue the remaining iterations (which would only idle on the flag).
 constexpr int kCgBlock = 8;
-hipError_t adj_pcg(const Batch& d, const AdjWork& A, int max_cg, double tol, hipStream_t s) {
-  auto vec = [&](int op) {
-    return launch_adj_vec(d, A.x, A.r, A.z, A.p, A.y, A.ec, A.zc, A.acc, A.gd, A.sc, A.done, tol, A.nx, A.n6, op, s);
-  };
-  auto precond = [&]() {
-    hipError_t e = launch_adj_obs(d, 1, A.spts, A.sposes, A.r, nullptr, A.ec, nullptr, nullptr, nullptr, nullptr, A.done, s);
-    if (e == hipSuccess) e = launch_adj_chol(A.Linv, A.n6, A.ec, A.zc, A.done, s);
-    if (e == hipSuccess)
-      e = launch_adj_obs(d, 2, A.spts, A.sposes, nullptr, A.acc, nullptr, A.zc, nullptr, nullptr, nullptr, A.done, s);
-    if (e == hipSuccess) e = vec(1);
-    return e;
-  };
-  hipError_t e = hipMemsetAsync(A.done, 0, sizeof(int32_t), s);
-  if (e == hipSuccess) e = vec(0);
-  if (e == hipSuccess) e = precond();
-  if (e == hipSuccess) e = vec(2);
+hipError_t adj_clear_done(const AdjData& A, hipStream_t s) { return launch_fill_zero(A.done, sizeof(int32_t), s); }
+
+hipError_t adj_pcg(const Batch& d, const AdjData& A, int max_cg, hipStream_t s) {
+  hipError_t e = adj_clear_done(A, s);
+  if (e == hipSuccess) e = launch_adj_start(d, A, s);
   int32_t done = 0;
   for (int it = 0; it < max_cg && e == hipSuccess && !done; ++it) {
-    e = launch_adj_obs(d, 0, A.spts, A.sposes, A.p, A.y, nullptr, nullptr, nullptr, nullptr, nullptr, A.done, s);
-    if (e == hipSuccess) e = vec(3);
-    if (e == hipSuccess) e = precond();
-    if (e == hipSuccess) e = vec(4);
+    e = launch_adj_iteration(d, A, it, s);
     if (e == hipSuccess && (it + 1) % kCgBlock == 0 && it + 1 < max_cg) {
       e = hipMemcpyAsync(&done, A.done, sizeof(done), hipMemcpyDeviceToHost, s);
       if (e == hipSuccess) e = hipStreamSynchronize(s);
     }
   }
-  return e;
-}
-
-// z = M^-1 gd with the factored Gauss-Newton preconditioner M = 2 sum rho' J^T L J (one application, no
-// conjugate gradients): a Gauss-Newton step.
-hipError_t adj_gn_step(const Batch& d, const AdjWork& A, hipStream_t s) {
-  hipError_t e = hipMemsetAsync(A.done, 0, sizeof(int32_t), s);
-  if (e == hipSuccess)
-    e = launch_adj_vec(d, A.x, A.r, A.z, A.p, A.y, A.ec, A.zc, A.acc, A.gd, A.sc, A.done, 0.0, A.nx, A.n6, 0, s);
-  if (e == hipSuccess)
-    e = launch_adj_obs(d, 1, A.spts, A.sposes, A.r, nullptr, A.ec, nullptr, nullptr, nullptr, nullptr, A.done, s);
-  if (e == hipSuccess) e = launch_adj_chol(A.Linv, A.n6, A.ec, A.zc, A.done, s);
-  if (e == hipSuccess)
-    e = launch_adj_obs(d, 2, A.spts, A.sposes, nullptr, A.acc, nullptr, A.zc, nullptr, nullptr, nullptr, A.done, s);
-  if (e == hipSuccess)
-    e = launch_adj_vec(d, A.x, A.r, A.z, A.p, A.y, A.ec, A.zc, A.acc, A.gd, A.sc, A.done, 0.0, A.nx, A.n6, 1, s);
-  return e;
-}
-
-// gd = gradient of the cost at the FP64 state.
-hipError_t adj_grad(const Batch& d, const AdjWork& A, hipStream_t s) {
-  hipError_t e = hipMemsetAsync(A.gd, 0, sizeof(double) * A.nx, s);
-  if (e == hipSuccess)
-    e = launch_adj_obs(d, 4, A.spts, A.sposes, nullptr, A.gd, nullptr, nullptr, nullptr, nullptr, nullptr, A.done, s);
   return e;
 }
 
@@ -1867,7 +1841,8 @@ int sba_batch_refine(sba_handle* h, sba_batch* b, int32_t gauss_newton_steps, in
   if (!h || !b || gauss_newton_steps < 0 || newton_steps < 0 || max_cg < 1)
     return fail(h, SBA_E_INVALID, "bad sba_batch_refine arguments");
   HIP_TRY(hipSetDevice(h->opt.device));
-  AdjWork A{};
+  AdjData A{};
+  A.tol = tol;
   int rc = adj_prepare(h, b, A);
   if (rc != SBA_OK) return rc;
   const Batch d = b->dev;
@@ -1875,19 +1850,20 @@ int sba_batch_refine(sba_handle* h, sba_batch* b, int32_t gauss_newton_steps, in
   hipStream_t s = h->stream;
   // Gauss-Newton steps x <- x - M^-1 grad: the factored system is positive definite, so these descend safely
   // from where the FP32 solve stopped, into the region where the full Hessian is positive definite too
-  for (int k = 0; k < gauss_newton_steps; ++k) {
-    HIP_TRY(adj_grad(d, A, s));
-    HIP_TRY(adj_gn_step(d, A, s));
+  for (int k = 0; k < gauss_newton_steps; ++k) {  // one application of the preconditioner
+    HIP_TRY(launch_adj_assemble(d, A, false, s));
+    HIP_TRY(adj_clear_done(A, s));
+    HIP_TRY(launch_adj_start(d, A, s));
     HIP_TRY(launch_adj_state(d, A.spts, A.sposes, A.z, 1, s));
   }
   // Newton steps x <- x - H^-1 grad, full FP64 Hessian, the stored factor as preconditioner
   for (int k = 0; k < newton_steps; ++k) {
-    HIP_TRY(adj_grad(d, A, s));
-    HIP_TRY(adj_pcg(d, A, max_cg, tol, s));
+    HIP_TRY(launch_adj_assemble(d, A, true, s));
+    HIP_TRY(adj_pcg(d, A, max_cg, s));
     HIP_TRY(launch_adj_state(d, A.spts, A.sposes, A.x, 1, s));
   }
   if (grad_norm) {
-    HIP_TRY(adj_grad(d, A, s));
+    HIP_TRY(launch_adj_assemble(d, A, false, s));
     std::vector<double> g(A.nx);
     HIP_TRY(hipMemcpyAsync(g.data(), A.gd, sizeof(double) * A.nx, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
@@ -2066,22 +2042,24 @@ int sba_batch_adjoint(sba_handle* h, sba_batch* b, const double* g, double* dxy,
                       double tol, int32_t* cg_iterations, double* a_out) {
   if (!h || !b || !g || !dxy || !dinfo || max_cg < 1) return fail(h, SBA_E_INVALID, "bad sba_batch_adjoint arguments");
   HIP_TRY(hipSetDevice(h->opt.device));
-  AdjWork A{};
+  AdjData A{};
+  A.tol = tol;
   int rc = adj_prepare(h, b, A);
   if (rc != SBA_OK) return rc;
   const Batch d = b->dev;
   hipStream_t s = h->stream;
+  HIP_TRY(launch_adj_assemble(d, A, true, s));
   HIP_TRY(hipMemcpyAsync(A.gd, g, sizeof(double) * A.nx, hipMemcpyHostToDevice, s));
-  HIP_TRY(adj_pcg(d, A, max_cg, tol, s));
+  HIP_TRY(adj_pcg(d, A, max_cg, s));
   // per-observation gradients from the adjoint
-  HIP_TRY(launch_adj_obs(d, 3, A.spts, A.sposes, A.x, nullptr, nullptr, nullptr, A.dxy, A.dinfo, b->obs_orig, A.done, s));
+  HIP_TRY(launch_adj_obs_grad(d, A, b->obs_orig, s));
   double scal[8];
   HIP_TRY(hipMemcpyAsync(scal, A.sc, sizeof(scal), hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipMemcpyAsync(dxy, A.dxy, sizeof(double) * 2 * A.no, hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipMemcpyAsync(dinfo, A.dinfo, sizeof(double) * 3 * A.no, hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipMemcpyAsync(dxy, A.dxy, sizeof(double) * 2 * b->win[0].no, hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipMemcpyAsync(dinfo, A.dinfo, sizeof(double) * 3 * b->win[0].no, hipMemcpyDeviceToHost, s));
   if (a_out) HIP_TRY(hipMemcpyAsync(a_out, A.x, sizeof(double) * A.nx, hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
-  if (cg_iterations) *cg_iterations = static_cast<int32_t>(scal[3]);
+  if (cg_iterations) *cg_iterations = static_cast<int32_t>(scal[2]);
   return SBA_OK;
 }
 
