@@ -274,7 +274,7 @@ __host__ __device__ inline bool inverse3(const double* m, double* out, double th
 // The control state of one window's solve, shared by the workgroup (LDS on the GPU).
 struct MonoShared {
   double residual, old, lambda, red[kMonoThreads];
-  int32_t count, new_values, failed, feasible, iteration, ok, total, n, stop, chol, ired[kMonoThreads];
+  int32_t count, new_values, failed, feasible, iteration, ok, total, n, stop, ired[kMonoThreads];
 };
 
 // ---- the solver: one workgroup per window -------------------------------------------------------------------------
@@ -314,15 +314,43 @@ struct MonoSolve {
   __host__ __device__ int isum(int v) {
     sh.ired[tid] = v;
     MONO_SYNC();
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (tid < 64) {
+      int s = (sh.ired[tid] + sh.ired[tid + 64]) + (sh.ired[tid + 128] + sh.ired[tid + 192]);
+      for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+      if (tid == 0) sh.ired[0] = s;
+    }
+#else
     if (tid == 0) {
       int s = 0;
       for (int i = 0; i < nth; ++i) s += sh.ired[i];
       sh.ired[0] = s;
     }
+#endif
     MONO_SYNC();
     const int s = sh.ired[0];
     MONO_SYNC();
     return s;
+  }
+
+  // workgroup maximum of v >= 0
+  __host__ __device__ double max(double v) {
+    sh.red[tid] = v;
+    MONO_SYNC();
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (tid < 64) {
+      double m = fmax(fmax(sh.red[tid], sh.red[tid + 64]), fmax(sh.red[tid + 128], sh.red[tid + 192]));
+      for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
+      if (tid == 0) sh.red[0] = m;
+    }
+#else
+    if (tid == 0)
+      for (int i = 1; i < nth; ++i) sh.red[0] = sh.red[i] > sh.red[0] ? sh.red[i] : sh.red[0];
+#endif
+    MONO_SYNC();
+    const double m = sh.red[0];
+    MONO_SYNC();
+    return m;
   }
 
   // Sliced sums: `items` independent sums (frames, reduced-system blocks), each over a list of terms, are split
@@ -698,29 +726,20 @@ struct MonoSolve {
   }
 
   // In-place Cholesky A = L L^T (lower triangle) of the n x n row-major A, right-looking by columns; false on a
-  // non-positive pivot.
+  // non-positive pivot. Two barriers per column: every thread reads the pivot and takes its square root itself, and the
+  // trailing triangle is walked by a 16 x 16 grid of the workgroup's threads (the barriers bound it; n is 30 for a
+  // tracker's window).
   __host__ __device__ bool cholesky(int n, double* A) {
-    if (tid == 0) sh.chol = 1;
-    MONO_SYNC();
+    const int cols = nth >= 256 ? 16 : 1, rows = nth / cols, ti = tid / cols, tj = tid % cols;
     for (int k = 0; k < n; ++k) {
-      if (tid == 0) {
-        const double d = A[k * n + k];
-        if (!(d > 0.0)) sh.chol = 0;
-        A[k * n + k] = d > 0.0 ? sqrt(d) : 1.0;
-      }
-      MONO_SYNC();
-      if (!sh.chol) return false;
-      const double dk = A[k * n + k];
+      const double d = A[k * n + k];
+      if (!(d > 0.0)) return false;  // the same value in every thread; the callers start with a barrier
+      const double dk = sqrt(d);
       for (int i = k + 1 + tid; i < n; i += nth) A[i * n + k] /= dk;
       MONO_SYNC();
-      const int m = n - k - 1;  // trailing lower triangle, row-major over (i, j), k < j <= i
-      for (int e = tid; e < m * (m + 1) / 2; e += nth) {
-        int i = static_cast<int>((sqrt(8.0 * e + 1.0) - 1.0) * 0.5);
-        while (i * (i + 1) / 2 > e) --i;
-        while ((i + 1) * (i + 2) / 2 <= e) ++i;
-        const int j = e - i * (i + 1) / 2;
-        A[(k + 1 + i) * n + (k + 1 + j)] -= A[(k + 1 + i) * n + k] * A[(k + 1 + j) * n + k];
-      }
+      for (int i = k + 1 + ti; i < n; i += rows)
+        for (int j = k + 1 + tj; j <= i; j += cols) A[i * n + j] -= A[i * n + k] * A[j * n + k];
+      if (tid == 0) A[k * n + k] = dk;
       MONO_SYNC();
     }
     return true;
@@ -741,22 +760,19 @@ struct MonoSolve {
       for (int j = 0; j < n; ++j) r += fabs(w.S[i * n + j]);
       rmax = r > rmax ? r : rmax;
     }
-    sh.red[tid] = rmax;
-    MONO_SYNC();
-    if (tid == 0) {
-      double m = 0.0;
-      for (int i = 0; i < nth; ++i) m = sh.red[i] > m ? sh.red[i] : m;
-      sh.red[0] = m;
-    }
-    MONO_SYNC();
-    const double tau = double(n) * kFltEps * sh.red[0];
-    MONO_SYNC();
+    const double tau = double(n) * kFltEps * max(rmax);
     for (int e = tid; e < nn; e += nth) A[e] = w.S[e] - (e / n == e % n ? tau : 0.0);
     MONO_SYNC();
-    if (!cholesky(n, A)) return nullptr;
+    if (!cholesky(n, A)) {
+      MONO_SYNC();  // every thread has read the pivot
+      return nullptr;
+    }
     for (int e = tid; e < nn; e += nth) A[e] = w.S[e];
     MONO_SYNC();
-    if (!cholesky(n, A)) return nullptr;
+    if (!cholesky(n, A)) {
+      MONO_SYNC();
+      return nullptr;
+    }
     return A;
   }
 
@@ -776,6 +792,57 @@ struct MonoSolve {
     }
     MONO_SYNC();
   }
+
+#if defined(__HIP_DEVICE_COMPILE__)
+  // The refined solve below by one wavefront for n <= 64 and a factor in workgroup memory: lane i keeps entry i of every
+  // vector in registers, the factor's columns and a transposed copy of S (St) in workgroup memory, and a solved entry is
+  // broadcast to the other lanes, so there is neither a barrier nor a dependent memory access in a substitution step
+  // (by one thread through global memory, the five solves of a step were most of the solver's time). No one but lanes
+  // of the first wavefront may call it.
+  __device__ double lane_bcast(double v, int j) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), j),
+                            __builtin_amdgcn_readlane(__double2loint(v), j));
+  }
+  __device__ void solve_by_wavefront(int n, const double* L, const double* St) {
+    const int i = tid < n ? tid : n - 1;  // lanes past n repeat the last row and are not stored
+    const bool in = tid < n;
+    const double b = in ? w.Sb[i] : 0.0, dii = L[i * n + i];
+    double xt = 0.0, x = 0.0, bd = b;
+    auto norm2 = [&](double v) {
+      double s = in ? v * v : 0.0;
+      for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+      return sqrt(s);
+    };
+    double min_norm = 1.79769313486231570e+308, nrm = norm2(b);
+    for (int it = 0; nrm < min_norm && it < 5; ++it) {
+      min_norm = nrm;
+      x = xt;
+      double v = bd;
+      for (int j = 0; j < n; ++j) {  // L y = bd, by columns
+        const double lij = L[i * n + j];
+        if (i == j) v /= dii;
+        const double y = lane_bcast(v, j);
+        if (i > j) v -= lij * y;
+      }
+      for (int j = n - 1; j >= 0; --j) {  // L^T d = y
+        const double lji = L[j * n + i];
+        if (i == j) v /= dii;
+        const double d = lane_bcast(v, j);
+        if (i < j) v -= lji * d;
+      }
+      xt += v;
+      double r = b;
+      for (int j = 0; j < n; ++j) r -= St[j * n + i] * lane_bcast(xt, j);
+      bd = r;
+      nrm = norm2(bd);
+      if (nrm < kFltEps) {
+        x = xt;
+        break;
+      }
+    }
+    if (in) w.x[i] = x;
+  }
+#endif
 
   // out = Q diag(1/ev) Q^T rhs
   __host__ __device__ void psolve(int n, const double* rhs, double* out) {
@@ -797,6 +864,41 @@ struct MonoSolve {
     double s = 0.0;
     for (int i = tid; i < n; i += nth) s += v[i] * v[i];
     return sqrt(sum(s));
+  }
+
+  // IterativeSolver: up to five steps x += solve(b - S x), kept while the residual norm decreases
+  __host__ __device__ void solve_refined(int n, const double* L) {
+    for (int i = tid; i < n; i += nth) {
+      w.xt[i] = 0.0;
+      w.bd[i] = w.Sb[i];
+      w.x[i] = 0.0;
+    }
+    MONO_SYNC();
+    double min_norm = 1.79769313486231570e+308;
+    double nrm = norm(n, w.Sb);
+    for (int it = 0; nrm < min_norm && it < 5; ++it) {
+      min_norm = nrm;
+      for (int i = tid; i < n; i += nth) w.x[i] = w.xt[i];
+      MONO_SYNC();
+      if (L)
+        chol_solve(n, L, w.bd, w.dv);
+      else
+        psolve(n, w.bd, w.dv);
+      for (int i = tid; i < n; i += nth) w.xt[i] += w.dv[i];
+      MONO_SYNC();
+      for (int i = tid; i < n; i += nth) {
+        double s = w.Sb[i];
+        for (int j = 0; j < n; ++j) s -= w.S[i * n + j] * w.xt[j];
+        w.bd[i] = s;
+      }
+      MONO_SYNC();
+      nrm = norm(n, w.bd);
+      if (nrm < kFltEps) {
+        for (int i = tid; i < n; i += nth) w.x[i] = w.xt[i];
+        MONO_SYNC();
+        break;
+      }
+    }
   }
 
   // The reduced system, its solve and the back-substitution (mono_sba_solver.cpp:681-702, 812-890): false when no
@@ -897,38 +999,17 @@ struct MonoSolve {
       MONO_SYNC();
       if (!sh.ok) return false;
     }
-    // IterativeSolver: up to five steps x += solve(b - S x), kept while the residual norm decreases
-    for (int i = tid; i < n; i += nth) {
-      w.xt[i] = 0.0;
-      w.bd[i] = w.Sb[i];
-      w.x[i] = 0.0;
-    }
-    MONO_SYNC();
-    double min_norm = 1.79769313486231570e+308;
-    double nrm = norm(n, w.Sb);
-    for (int it = 0; nrm < min_norm && it < 5; ++it) {
-      min_norm = nrm;
-      for (int i = tid; i < n; i += nth) w.x[i] = w.xt[i];
+#if defined(__HIP_DEVICE_COMPILE__)
+    const bool by_wavefront = L != nullptr && L == lds && n <= 64 && 2 * static_cast<int64_t>(n) * n <= lds_cap;
+    if (by_wavefront) {  // workgroup-uniform
+      double* St = lds + n * n;
+      for (int e = tid; e < n * n; e += nth) St[(e % n) * n + e / n] = w.S[e];
       MONO_SYNC();
-      if (L)
-        chol_solve(n, L, w.bd, w.dv);
-      else
-        psolve(n, w.bd, w.dv);
-      for (int i = tid; i < n; i += nth) w.xt[i] += w.dv[i];
+      if (tid < 64) solve_by_wavefront(n, L, St);
       MONO_SYNC();
-      for (int i = tid; i < n; i += nth) {
-        double s = w.Sb[i];
-        for (int j = 0; j < n; ++j) s -= w.S[i * n + j] * w.xt[j];
-        w.bd[i] = s;
-      }
-      MONO_SYNC();
-      nrm = norm(n, w.bd);
-      if (nrm < kFltEps) {
-        for (int i = tid; i < n; i += nth) w.x[i] = w.xt[i];
-        MONO_SYNC();
-        break;
-      }
-    }
+    } else
+#endif
+      solve_refined(n, L);
     for (int f = tid; f < w.nF; f += nth)
       for (int i = 0; i < 6; ++i) w.fda[6 * f + i] = w.constrained[f] ? 0.0 : w.x[6 * w.free_idx[f] + i];
     MONO_SYNC();
