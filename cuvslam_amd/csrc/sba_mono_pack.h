@@ -6,7 +6,6 @@
 
 #include <algorithm>
 #include <cstdint>
-#include <numeric>
 #include <vector>
 
 #include "../../include/cuvslam_sba_mono.h"
@@ -33,22 +32,34 @@ inline bool pack_window(const sba_mono_window& v, MonoPack& k) {
   k.otrack.assign(v.obs_track, v.obs_track + k.nO);
   for (int o = 0; o < k.nO; ++o)
     if (k.oframe[o] < 0 || k.oframe[o] >= k.nF || k.otrack[o] < 0 || k.otrack[o] >= k.nT) return false;
-  std::vector<int32_t> idx(k.nO);
-  std::iota(idx.begin(), idx.end(), 0);
-  k.tobs = idx;
-  std::stable_sort(k.tobs.begin(), k.tobs.end(), [&](int a, int b) {
-    return k.otrack[a] != k.otrack[b] ? k.otrack[a] < k.otrack[b] : k.oframe[a] < k.oframe[b];
-  });
-  k.fobs = idx;
-  std::stable_sort(k.fobs.begin(), k.fobs.end(), [&](int a, int b) {
-    return k.oframe[a] != k.oframe[b] ? k.oframe[a] < k.oframe[b] : k.otrack[a] < k.otrack[b];
-  });
   k.track_obs.assign(k.nT + 1, 0);
   for (int o = 0; o < k.nO; ++o) ++k.track_obs[k.otrack[o] + 1];
   for (int t = 0; t < k.nT; ++t) k.track_obs[t + 1] += k.track_obs[t];
   k.frame_obs.assign(k.nF + 1, 0);
   for (int o = 0; o < k.nO; ++o) ++k.frame_obs[k.oframe[o] + 1];
   for (int f = 0; f < k.nF; ++f) k.frame_obs[f + 1] += k.frame_obs[f];
+  // stable counting sorts: by frame and then by track (a track's observations in frame order), and the other way round
+  k.tobs.resize(k.nO);
+  k.fobs.resize(k.nO);
+  std::vector<int32_t> pass(k.nO), next;
+  auto by_frame = [&](const int32_t* src, int32_t* dst) {
+    next.assign(k.frame_obs.begin(), k.frame_obs.end() - 1);
+    for (int i = 0; i < k.nO; ++i) {
+      const int o = src ? src[i] : i;
+      dst[next[k.oframe[o]]++] = o;
+    }
+  };
+  auto by_track = [&](const int32_t* src, int32_t* dst) {
+    next.assign(k.track_obs.begin(), k.track_obs.end() - 1);
+    for (int i = 0; i < k.nO; ++i) {
+      const int o = src ? src[i] : i;
+      dst[next[k.otrack[o]]++] = o;
+    }
+  };
+  by_frame(nullptr, pass.data());
+  by_track(pass.data(), k.tobs.data());
+  by_track(nullptr, pass.data());
+  by_frame(pass.data(), k.fobs.data());
   // ordered pairs (j, k) of every track's free frames, per block in track order
   const int nb = k.nFree * k.nFree;
   k.blk.assign(nb + 1, 0);

@@ -6,7 +6,9 @@
 #include <algorithm>
 #include <cstdint>
 #include <cstring>
+#include <new>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/cuvslam_sba_mono.h"
@@ -25,12 +27,18 @@ namespace {
 constexpr int64_t kMonoLds = 18432;  // doubles of workgroup memory (144 KiB): 3 n^2 for n <= 78 (13 free frames)
 constexpr int kMaxMonoFree = 64;  // free frames per window: reduced system of order <= 384
 
-struct Slab {  // host staging of everything a batch uploads, with the device offset of each piece
-  std::vector<char> bytes;
+// Every piece that a batch uploads, at its offset of one staging buffer and of the device block.
+struct Slab {
+  struct Piece {
+    const void* src;
+    size_t off, bytes;
+  };
+  std::vector<Piece> pieces;
+  size_t total = 0;
   size_t add(const void* src, size_t n) {
-    const size_t o = bytes.size();
-    bytes.resize(o + ((n + 255) & ~size_t(255)));
-    if (n && src) std::memcpy(bytes.data() + o, src, n);
+    const size_t o = total;
+    if (n && src) pieces.push_back(Piece{src, o, n});
+    total += (n + 255) & ~size_t(255);
     return o;
   }
 };
@@ -61,14 +69,30 @@ int sba_mono_solve_batch(sba_handle* h, const sba_mono_window* windows, int32_t 
     size_t con, fidx, pose, fro, fob, pts, tro, tob, ofr, otr, oxy, blk, bpr;
   };
   std::vector<Offs> offs(n);
-  for (int i = 0; i < n; ++i) {
+  // windows are packed on the handle's host threads, one window each at a time (one after another the packing of 256
+  // windows took three quarters of the call); the checks keep their order
+  const int threads = static_cast<int>(std::min(16u, std::max(1u, std::thread::hardware_concurrency())));
+  std::vector<uint8_t> state(n, 0);  // 1 bad sizes or null buffers, 2 indexes out of range, 3 out of memory
+  sba_internal::parallel_for(h, n, threads, [&](int i) {
     const sba_mono_window& v = windows[i];
     if (v.num_frames < 0 || v.num_tracks < 0 || v.num_obs < 0 ||
         (v.num_frames && (!v.constrained || !v.frame_poses)) || (v.num_tracks && !v.points) ||
         (v.num_obs && (!v.obs_frame || !v.obs_track || !v.obs_xy)))
+      state[i] = 1;
+    else
+      try {
+        if (!pack_window(v, packs[i])) state[i] = 2;
+      } catch (const std::bad_alloc&) {  // must not leave a pool thread
+        state[i] = 3;
+      }
+  });
+  for (int i = 0; i < n; ++i) {
+    const sba_mono_window& v = windows[i];
+    if (state[i] == 1)
       return set_error(h, SBA_E_INVALID, "window " + std::to_string(i) + ": bad sizes or null buffers");
-    if (!pack_window(v, packs[i]))
+    if (state[i] == 2)
       return set_error(h, SBA_E_INVALID, "window " + std::to_string(i) + ": observation indexes out of range");
+    if (state[i] == 3) return set_error(h, SBA_E_INVALID, "out of host memory while packing");
     if (packs[i].nFree > kMaxMonoFree)
       return set_error(h, SBA_E_CAPACITY, "window " + std::to_string(i) + " has " + std::to_string(packs[i].nFree) +
                                               " free frames; at most " + std::to_string(kMaxMonoFree));
@@ -91,7 +115,7 @@ int sba_mono_solve_batch(sba_handle* h, const sba_mono_window* windows, int32_t 
   // work areas (doubles unless noted), then every window's outputs in one region (read back with one copy):
   // scalars (8 doubles), covariance (36 doubles), poses (16 floats per frame), points (3 floats per track)
   std::vector<size_t> work(n), outp(n);
-  size_t total = in.bytes.size();
+  size_t total = in.total;
   auto round = [](size_t b) { return (b + 255) & ~size_t(255); };
   constexpr size_t kResHead = 64 + 288;
   std::vector<size_t> wbytes(n);
@@ -167,7 +191,16 @@ int sba_mono_solve_batch(sba_handle* h, const sba_mono_window* windows, int32_t 
     jobs[i].poses_out = reinterpret_cast<float*>(r + kResHead);
     jobs[i].pts_out = reinterpret_cast<float*>(r + kResHead + 64 * F);
   }
-  hipError_t e = hipMemcpyAsync(base, in.bytes.data(), in.bytes.size(), hipMemcpyHostToDevice, st);
+  // staged in page-locked memory that the handle keeps (the results' copy below waits for the stream, so the buffer is
+  // free again when this returns)
+  char* stage = nullptr;
+  if (int rc = sba_internal::host_staging(h, std::max(in.total, res_bytes), &stage); rc != SBA_OK) return rc;
+  const int parts = static_cast<int>(in.pieces.size());
+  sba_internal::parallel_for(h, std::min(parts, 64), in.total > (1 << 20) ? threads : 1, [&](int c) {
+    for (int k = parts * c / std::min(parts, 64); k < parts * (c + 1) / std::min(parts, 64); ++k)
+      std::memcpy(stage + in.pieces[k].off, in.pieces[k].src, in.pieces[k].bytes);
+  });
+  hipError_t e = hipMemcpyAsync(base, stage, in.total, hipMemcpyHostToDevice, st);
   if (e == hipSuccess)
     e = hipMemcpyAsync(base + jobs_off, jobs.data(), sizeof(MonoJob) * size_t(n), hipMemcpyHostToDevice, st);
   // workgroup memory for the eigen-decomposition of the largest reduced system, up to kMonoLds
@@ -179,16 +212,19 @@ int sba_mono_solve_batch(sba_handle* h, const sba_mono_window* windows, int32_t 
   if (lds > kMonoLds) lds = 0;  // the largest does not fit: every window keeps its matrices in its work area
   if (e == hipSuccess)
     e = launch_mono_solve(reinterpret_cast<const MonoJob*>(base + jobs_off), n, static_cast<int>(lds), st);
-  if (e != hipSuccess) return set_error(h, SBA_E_DEVICE, std::string("mono solve: ") + hipGetErrorString(e));
-  std::vector<char> host_res(res_bytes);
-  if (e == hipSuccess) e = hipMemcpyAsync(host_res.data(), base + res_base, res_bytes, hipMemcpyDeviceToHost, st);
+  if (e != hipSuccess) {
+    (void)hipStreamSynchronize(st);  // a copy that was enqueued may still read the staging
+    return set_error(h, SBA_E_DEVICE, std::string("mono solve: ") + hipGetErrorString(e));
+  }
+  // into the same staging: the upload is complete when the kernel, and so this copy, starts
+  if (e == hipSuccess) e = hipMemcpyAsync(stage, base + res_base, res_bytes, hipMemcpyDeviceToHost, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (e != hipSuccess) return set_error(h, SBA_E_DEVICE, std::string("mono results: ") + hipGetErrorString(e));
   double sc[8], cov[36];
   for (int i = 0; i < n; ++i) {
     const MonoPack& k = packs[i];
     sba_mono_result& r = results[i];
-    const char* src = host_res.data() + outp[i];
+    const char* src = stage + outp[i];
     std::memcpy(sc, src, 64);
     std::memcpy(cov, src + 64, 288);
     if (r.frame_poses && k.nF) std::memcpy(r.frame_poses, src + kResHead, 64 * size_t(k.nF));

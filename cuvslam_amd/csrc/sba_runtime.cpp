@@ -249,6 +249,9 @@ struct sba_handle {
   // device workspace of the inertial solve (sba_imu_solve), kept and regrown like ws
   char* imu_ws = nullptr;
   size_t imu_ws_bytes = 0;
+  // page-locked host staging of the mono solve
+  char* stage = nullptr;
+  size_t stage_bytes = 0;
 };
 
 struct sba_batch {
@@ -928,6 +931,7 @@ int sba_destroy(sba_handle* h) {
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   if (h->ws) (void)hipFree(h->ws);
   if (h->imu_ws) (void)hipFree(h->imu_ws);
+  if (h->stage) (void)hipHostFree(h->stage);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
   return SBA_OK;
@@ -962,6 +966,21 @@ int aux_workspace(sba_handle* h, size_t bytes, char** out) {
     h->imu_ws_bytes = grown;
   }
   *out = h->imu_ws;
+  return SBA_OK;
+}
+
+int host_staging(sba_handle* h, size_t bytes, char** out) {
+  if (bytes > h->stage_bytes) {
+    if (h->stage) {
+      HIP_TRY(hipStreamSynchronize(h->stream));
+      HIP_TRY(hipHostFree(h->stage));
+      h->stage = nullptr;
+      h->stage_bytes = 0;
+    }
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&h->stage), bytes, hipHostMallocDefault));
+    h->stage_bytes = bytes;
+  }
+  *out = h->stage;
   return SBA_OK;
 }
 
