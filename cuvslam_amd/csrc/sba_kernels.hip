@@ -822,21 +822,23 @@ __global__ __launch_bounds__(256) void k_reduce(Batch b) {
 //
 // S + lambda diag(U) (n = 6 x free key frames <= 240) is cut into 16 x 16 tiles; A = U^T U is factored as the
 // upper tiles U_JI (J <= I) in the FP64 matrix-core layout (element (4v + lane / 16, lane % 16) in register v
-// of the lane, i.e. 64 v + lane in row-major order): wavefronts 1..7 keep the off-diagonal tiles in registers,
-// wavefront 0 the diagonal tiles in LDS. Right-looking, per tile column K:
-//   panel     U_KI = X_KK A_KI with the inverse X_KK = U_KK^-T (4 MFMA 16x16x4), published to LDS, and the
-//             forward substitution e_I -= U_KI^T y_K;
-//   trailing  A_JI -= U_KJ^T U_KI for K < J <= I (4 MFMA each); wavefront 0 first updates (K+1, K+1) and
-//             factors it (one wavefront, pivots broadcast with readlane, then X_{K+1,K+1} by forward
-//             substitution), so the serial 16 x 16 factor overlaps the other wavefronts' updates; y_K = X_KK e_K
-//             is formed at the start of the next panel step. Two barriers per tile column.
-// Backward substitution U x = y per tile column: x_K = X_KK^T r_K, then r_J -= U_JK x_K by the tiles' owners.
+// of the lane, i.e. 64 v + lane in row-major order): wavefronts 1..7 keep the tiles with I > J + 1 in registers, the
+// diagonal tiles and the ones next to them (J, J + 1) lie in LDS. Right-looking, per tile column K:
+//   panel     U_KI = X_KK A_KI with the inverse X_KK = U_KK^-T (4 MFMA 16x16x4), published to LDS: (K, K + 1) by
+//             wavefront 0, which also takes U^T U of it from tile (K + 1, K + 1), the others by their owners;
+//   trailing  A_JI -= U_KJ^T U_KI for K < J <= I (4 MFMA each) and the forward substitution y_K = X_KK e_K,
+//             e_I -= U_KI^T y_K by wavefronts 1..7, while wavefront 0 factors tile (K + 1, K + 1) (factor_tile).
+// Two barriers per tile column. Wavefront 0's chain bounds it: a panel product, an update and a 16 x 16 factor per column;
+// that it forms the one panel tile it needs itself takes the wait for the other wavefronts' panel out of the chain.
+// Backward substitution U x = y per tile column: wavefront 0 forms r_K -= U_{K,K+1} x_{K+1} and x_K = X_KK^T r_K while
+// the tiles' owners apply x_{K+1} to the rows above; one barrier per column. 28 free key frames (11 tile columns): 58 us,
+// 66 with every panel tile formed by its owner and the backward row updates in one chain with x_K.
 // (Golub & Van Loan, Matrix Computations, 4.2.4 block Cholesky and 3.1 triangular systems.)
 // ---------------------------------------------------------------------------------------------------------
 namespace {
 
 constexpr int kFT = 15;     // tile rows of the largest reduced system (240 = 15 x 16)
-constexpr int kSlots = 15;  // register tiles per wavefront: 7 wavefronts hold the <= 105 off-diagonal tiles
+constexpr int kSlots = 13;  // register tiles per wavefront: 7 wavefronts hold the <= 91 tiles past the first off-diagonal
 
 __device__ __forceinline__ int64_t pk(int i, int j) { return static_cast<int64_t>(i) * (i + 1) / 2 + j; }
 
@@ -853,6 +855,7 @@ __global__ __launch_bounds__(kFactorThreads) void k_factor(Batch b, double* dbg_
   __shared__ double sDg[kFT * 256];   // diagonal tiles (wavefront 0), row-major
   __shared__ double sXT[kFT * 256];   // X_KK^T of every tile column
   __shared__ double sP[kFT * 256];    // panel tiles U_KI of the current tile column
+  __shared__ double sUp[(kFT - 1) * 256];  // tiles (J, J + 1), row-major
   __shared__ int flag;
   const int w = blockIdx.x;
   const WindowDesc W = b.win[w];
@@ -912,16 +915,27 @@ __global__ __launch_bounds__(kFactorThreads) void k_factor(Batch b, double* dbg_
     if (i < n && j <= i) store_L[pk(i, j)] = val;
   };
 
-  // the diagonal tiles, kept in LDS, are assembled by all wavefronts
-  for (int J = wave; J < T; J += kFactorThreads / 64) {
+  // y_K = X_KK e_K, lane l holds y_K[l % 16]
+  auto forward = [&](int K) {
+    const double* xt = sXT + 256 * K;
+    double yk = 0.0;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) yk += xt[16 * (4 * li + kk) + lj] * vec[16 * K + 4 * li + kk];
+    return sum_rows4(yk);
+  };
+
+  // the tiles kept in LDS, (m / 2, (m + 1) / 2) for m = 0 .. 2 T - 2, are assembled by all wavefronts
+  for (int m = wave; m < 2 * T - 1; m += kFactorThreads / 64) {
+    const int J = m / 2, I = (m + 1) / 2;
+    double* dst = J == I ? sDg + 256 * J : sUp + 256 * J;
     double val[4];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) val[v] = element(J, J, v);
+    for (int v = 0; v < 4; ++v) val[v] = element(J, I, v);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) sDg[256 * J + 64 * v + lane] = val[v];
+    for (int v = 0; v < 4; ++v) dst[64 * v + lane] = val[v];
     if (dbg_S && w == 0) {
 #pragma unroll
-      for (int v = 0; v < 4; ++v) dbg_tile(J, J, v, val[v]);
+      for (int v = 0; v < 4; ++v) dbg_tile(J, I, v, val[v]);
     }
   }
 
@@ -930,63 +944,82 @@ __global__ __launch_bounds__(kFactorThreads) void k_factor(Batch b, double* dbg_
     __syncthreads();
     // 2. factorization; K = -1 only factors tile (0, 0). The other wavefronts run their own copy of the loop
     //    with the same barriers.
-    for (int K = -1; K < T; ++K) {
+    for (int K = -1; K + 1 < T; ++K) {
       if (flag) break;
+      double* tk = sDg + 256 * (K + 1);
+      double4v dt;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) dt[v] = tk[64 * v + lane];
       if (K >= 0) {
         const double* xt = sXT + 256 * K;
-        double yk = 0.0;  // y_K = X_KK e_K
+        double* up = sUp + 256 * K;
+        double4v u = double4v{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) yk += xt[16 * (4 * li + kk) + lj] * vec[16 * K + 4 * li + kk];
-        yk = sum_rows4(yk);
-        if (lane < 16) ys[16 * K + lane] = yk;
+        for (int q = 0; q < 4; ++q) u = mfma64(xt[64 * q + lane], up[64 * q + lane], u);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          sP[256 * (K + 1) + 64 * v + lane] = u[v];
+          up[64 * v + lane] = u[v];
+        }
+        // the registers of u are both operands of u^T u
+#pragma unroll
+        for (int q = 0; q < 4; ++q) dt = mfma64(-u[q], u[q], dt);
         __syncthreads();
       }
-      // the next diagonal tile first: update, factor; then the remaining diagonal tiles
-      if (K + 1 < T) {
-        double* tk = sDg + 256 * (K + 1);
-        double4v dt;
+      if (!factor_tile(dt, sXT + 256 * (K + 1), idg + 16 * (K + 1), lane) && lane == 0) flag = 1;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) dt[v] = tk[64 * v + lane];
-        if (K >= 0) dt = tile_update(dt, sP + 256 * (K + 1), sP + 256 * (K + 1), lane);
-        if (!factor_tile(dt, sXT + 256 * (K + 1), idg + 16 * (K + 1), lane) && lane == 0) flag = 1;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) tk[64 * v + lane] = dt[v];
-      }
+      for (int v = 0; v < 4; ++v) tk[64 * v + lane] = dt[v];
       __syncthreads();
     }
     if (keep) {
       for (int J = 0; J < T; ++J)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) keep_tile(J, J, v, sDg[256 * J + 64 * v + lane]);
+        for (int v = 0; v < 4; ++v) {
+          keep_tile(J, J, v, sDg[256 * J + 64 * v + lane]);
+          if (J + 1 < T) keep_tile(J, J + 1, v, sUp[256 * J + 64 * v + lane]);
+        }
     } else if (flag == 0) {
-      // 3. backward substitution U x = y, tile column K from T - 1 down: x_K = X_KK^T r_K (here), then
-      //    r_J -= U_JK x_K (the owners of (J, K))
+      // 3. backward substitution U x = y from the last tile column: r_K -= U_{K,K+1} x_{K+1}, x_K = X_KK^T r_K here,
+      //    then the owners take U_JK x_K from r_J, J < K - 1, while the next column is formed here. y_{T-1} first.
+      double xk = 0.0;  // x_{K+1}[lane % 16]
       for (int K = T - 1; K >= 0; --K) {
         const double* xt = sXT + 256 * K;
-        double p = 0.0;
+        double xv[4], p[4];
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) p += xt[16 * lj + 4 * li + kk] * ys[16 * K + 4 * li + kk];
-        p = sum_rows4(p);
-        if (lane < 16) xs[16 * K + lane] = p;
+        for (int v = 0; v < 4; ++v) xv[v] = xt[16 * lj + 4 * v + li];  // X_KK[4v + lane/16][lane%16]
+        if (K == T - 1) {
+          const double yk = forward(K);
+#pragma unroll
+          for (int v = 0; v < 4; ++v) p[v] = __shfl(yk, 4 * v + li);
+        } else {
+          const double* up = sUp + 256 * K;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) p[v] = ys[16 * K + 4 * v + li] - sum_row16_dpp(up[64 * v + lane] * xk);
+        }
+        double x = 0.0;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) x += xv[v] * p[v];
+        xk = sum_rows4(x);
+        if (lane < 16) xs[16 * K + lane] = xk;
         __syncthreads();
       }
     }
   } else {
-    // wavefronts 1..7: the off-diagonal tiles (J < I) in registers, tile m of the row-major order in slot
+    // wavefronts 1..7: the tiles (J, I), I > J + 1, in registers, tile m of the row-major order in slot
     // (m / 7) of wavefront 1 + m % 7
     int tJ[kSlots], tI[kSlots];
     {
-      const int noff = T * (T - 1) / 2;
+      const int noff = T > 2 ? (T - 1) * (T - 2) / 2 : 0;
 #pragma unroll
       for (int s = 0; s < kSlots; ++s) {
         int m = 7 * s + wave - 1, J = 0;
         if (m < noff) {
-          while (m >= T - 1 - J) {
-            m -= T - 1 - J;
+          while (m >= T - 2 - J) {
+            m -= T - 2 - J;
             ++J;
           }
           tJ[s] = J;
-          tI[s] = J + 1 + m;
+          tI[s] = J + 2 + m;
         } else {
           tJ[s] = -1;
           tI[s] = -1;
@@ -1010,19 +1043,11 @@ __global__ __launch_bounds__(kFactorThreads) void k_factor(Batch b, double* dbg_
           for (int v = 0; v < 4; ++v) dbg_tile(tJ[s], tI[s], v, acc[s][v]);
     }
     __syncthreads();
-    for (int K = -1; K < T; ++K) {
+    for (int K = -1; K + 1 < T; ++K) {
       if (flag) break;
       if (K >= 0) {
-        // panel U_KI = X_KK A_KI (the B operand of chunk q is register q of the tile itself), published to
-        // LDS, and e_I -= U_KI^T y_K
+        // panel U_KI = X_KK A_KI (the B operand of chunk q is register q of the tile itself), published to LDS
         const double* xt = sXT + 256 * K;
-        double yk = 0.0;
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) yk += xt[16 * (4 * li + kk) + lj] * vec[16 * K + 4 * li + kk];
-        yk = sum_rows4(yk);
-        double yv[4];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) yv[v] = __shfl(yk, 4 * v + li);  // y_K[4v + lane/16]
 #pragma unroll
         for (int s = 0; s < kSlots; ++s) {
           if (tJ[s] == K) {
@@ -1031,25 +1056,33 @@ __global__ __launch_bounds__(kFactorThreads) void k_factor(Batch b, double* dbg_
 #pragma unroll
             for (int q = 0; q < 4; ++q) u = mfma64(xt[64 * q + lane], acc[s][q], u);
             acc[s] = u;
-            double p = 0.0;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-              sP[256 * I + 64 * v + lane] = u[v];
-              p += u[v] * yv[v];
-            }
-            p = sum_rows4(p);
-            if (lane < 16) vec[16 * I + lane] -= p;
+            for (int v = 0; v < 4; ++v) sP[256 * I + 64 * v + lane] = u[v];
           }
         }
         __syncthreads();
-        // trailing A_JI -= U_KJ^T U_KI, K < J < I; and the diagonal tiles past K + 1 (in LDS), J = K + 2 + m
-        // by wavefront 1 + m % 7, while wavefront 0 factors tile K + 1
-        for (int J = K + 1 + wave; J < T; J += 7) {
-          double* tj = sDg + 256 * J;
+        // while wavefront 0 factors tile K + 1: y_K, and e_I -= U_KI^T y_K, I = K + 1 + m by wavefront 1 + m % 7
+        const double yk = forward(K);
+        if (wave == 1 && lane < 16) ys[16 * K + lane] = yk;
+        double yv[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) yv[v] = __shfl(yk, 4 * v + li);  // y_K[4v + lane/16]
+        for (int I = K + wave; I < T; I += 7) {
+          double p = 0.0;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) p += sP[256 * I + 64 * v + lane] * yv[v];
+          p = sum_rows4(p);
+          if (lane < 16) vec[16 * I + lane] -= p;
+        }
+        // trailing A_JI -= U_KJ^T U_KI: the LDS tiles past (K + 1, K + 1), tile m = 2 J + (I - J) > 2 K + 2 of the order
+        // above by wavefront 1 + (m - 2 K - 3) % 7, then the register tiles
+        for (int m = 2 * K + 2 + wave; m < 2 * T - 1; m += 7) {
+          const int J = m / 2, I = (m + 1) / 2;
+          double* tj = J == I ? sDg + 256 * J : sUp + 256 * J;
           double4v t;
 #pragma unroll
           for (int v = 0; v < 4; ++v) t[v] = tj[64 * v + lane];
-          t = tile_update(t, sP + 256 * J, sP + 256 * J, lane);
+          t = tile_update(t, sP + 256 * J, sP + 256 * I, lane);
 #pragma unroll
           for (int v = 0; v < 4; ++v) tj[64 * v + lane] = t[v];
         }
@@ -1070,19 +1103,18 @@ __global__ __launch_bounds__(kFactorThreads) void k_factor(Batch b, double* dbg_
           for (int v = 0; v < 4; ++v) keep_tile(tJ[s], tI[s], v, acc[s][v]);
     } else if (flag == 0) {
       for (int K = T - 1; K >= 0; --K) {
-        const double* xt = sXT + 256 * K;
-        double p = 0.0;
+        // x_{K+1} is published: apply it to the rows above K (row K is wavefront 0's), then meet it at x_K
+        if (K + 1 < T) {
+          const double p = xs[16 * (K + 1) + lj];
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) p += xt[16 * lj + 4 * li + kk] * ys[16 * K + 4 * li + kk];
-        p = sum_rows4(p);  // x_K[lane % 16]
+          for (int s = 0; s < kSlots; ++s) {
+            if (tI[s] == K + 1 && tJ[s] >= 0) {
+              const int J = in_loop(tJ[s]);
 #pragma unroll
-        for (int s = 0; s < kSlots; ++s) {
-          if (tI[s] == K && tJ[s] >= 0) {
-            const int J = in_loop(tJ[s]);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-              const double t = sum_row16_dpp(acc[s][v] * p);
-              if (lj == 0) ys[16 * J + 4 * v + li] -= t;
+              for (int v = 0; v < 4; ++v) {
+                const double t = sum_row16_dpp(acc[s][v] * p);
+                if (lj == 0) ys[16 * J + 4 * v + li] -= t;
+              }
             }
           }
         }
