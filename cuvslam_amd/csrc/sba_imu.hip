@@ -591,7 +591,9 @@ __global__ __launch_bounds__(kReducedThreads) void k_imu_reduced(Window w) {
     }
     __syncthreads();
     if (tid >= 256) return;
-    const int a = tid / 16, c = tid % 16;
+    // A diagonal block is its lower triangle mirrored: U and W are not symmetric where an observation's information
+    // matrix is not, and the factorization is defined on the lower triangle.
+    const int ra = tid / 16, rc = tid % 16, a = j == k ? max(ra, rc) : ra, c = j == k ? min(ra, rc) : rc;
     double* T = w.A + 256 * static_cast<int64_t>(blockIdx.x);  // lower tile (j, k), blocks in the same order
     if (a == 15 || c == 15) {  // padding: zero, and one on the diagonal of a diagonal tile
       T[tid] = (a == c && j == k) ? 1.0 : 0.0;
