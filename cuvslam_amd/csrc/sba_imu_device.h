@@ -21,7 +21,9 @@ namespace sba_imu_dev {
 constexpr int kThreads = 256;
 constexpr int kEdgeThreads = 256;  // one workgroup per inertial edge
 constexpr int kReducedThreads = 1024, kReducedSlices = 28;  // 36 x 28 partial sums per reduced block
-constexpr int kPoseFullThreads = 1024;  // 42 values x 24 slices of a key frame's reprojection sums
+constexpr int kPoseFullThreads = 512;  // a thread per observation of a key frame
+constexpr int kPointLanes = 8;         // lanes per point of the point kernels
+constexpr int kLdsTiles = 64;          // tiles of the reduced system's factor that fit in shared memory (128 KiB)
 constexpr int kFactorThreads = 512;
 constexpr int kMaxFree = 64;  // free key frames of one window (reduced system order <= 960)
 // one key frame's state: R (9, row-major), t (3), v (3), bg (3), ba (3)
@@ -95,6 +97,11 @@ struct Window {
   const int32_t* blk_jk;     // [nblocks][2] (j, k), j >= k
   const int32_t* blk_tri;    // [nblocks+1]
   const int2* tri;           // (pair of j, pair of k)
+  // tiles of the reduced system's factor that are not structurally zero: their number, each block's slot (-1: zero) and
+  // each slot's block
+  int32_t nslots;
+  const int32_t* blk_slot;   // [nblocks]
+  const int32_t* slot_blk;   // [nslots]
   const Preint* pre;         // [K]
   // state: [0] current, [1] trial
   double* pts[2];   // [P][3]

@@ -354,7 +354,7 @@ struct Packed {
   int P, N, K, F, n, C, npairs, nblocks;
   std::vector<double> xy, info, cam, pts, pose;
   std::vector<int32_t> opid, okid, ocid, point_obs, pobs, point_pair, pair_obs, pair_pose, pair_point, pose_obs, kobs,
-      pose_pair, kpair, blk_jk, blk_tri;
+      pose_pair, kpair, blk_jk, blk_tri, blk_slot, slot_blk;
   std::vector<int2> tri;
 };
 
@@ -505,6 +505,27 @@ void pack(const sba_imu_calibration& calib, const sba_imu_problem_view& v, Packe
         ++k.blk_tri[j * (j + 1) / 2 + q + 1];
       }
   for (int b = 0; b < k.nblocks; ++b) k.blk_tri[b + 1] += k.blk_tri[b];
+  // the tiles of the reduced system's Cholesky factor that are not structurally zero: blocks with common points, key
+  // frames that an inertial edge couples, and the fill-in of the elimination in key frame order
+  {
+    auto index = [](int i, int j) { return i * (i + 1) / 2 + j; };
+    std::vector<uint8_t> set(k.nblocks, 0);
+    for (int j = 0; j < k.n; ++j)
+      for (int q = 0; q <= j; ++q)
+        set[index(j, q)] = j - q <= 1 || k.blk_tri[index(j, q) + 1] > k.blk_tri[index(j, q)];
+    for (int c = 0; c < k.n; ++c)
+      for (int a = c + 1; a < k.n; ++a)
+        if (set[index(a, c)])
+          for (int b = c + 1; b <= a; ++b)
+            if (set[index(b, c)]) set[index(a, b)] = 1;
+    k.blk_slot.assign(std::max(k.nblocks, 1), -1);
+    k.slot_blk.clear();
+    for (int b = 0; b < k.nblocks; ++b)
+      if (set[b]) {
+        k.blk_slot[b] = int32_t(k.slot_blk.size());
+        k.slot_blk.push_back(b);
+      }
+  }
   k.tri.resize(std::max<size_t>(k.blk_tri[k.nblocks], 1));
   {
     std::vector<int32_t> fill(k.blk_tri.begin(), k.blk_tri.end() - 1);
@@ -628,6 +649,7 @@ int sba_imu_solve(sba_handle* h, const sba_imu_calibration* calib, const sba_imu
   const size_t o_pose_pair = L.add<int32_t>(k.pose_pair.size()), o_kpair = L.add<int32_t>(k.kpair.size());
   const size_t o_blk_jk = L.add<int32_t>(k.blk_jk.size()), o_blk_tri = L.add<int32_t>(k.blk_tri.size());
   const size_t o_tri = L.add<int2>(k.tri.size());
+  const size_t o_blk_slot = L.add<int32_t>(k.blk_slot.size()), o_slot_blk = L.add<int32_t>(k.slot_blk.size());
   const size_t o_pre = L.add<Preint>(k.K);
   const size_t o_pts0 = L.add<double>(3 * size_t(k.P)), o_pts1 = L.add<double>(3 * size_t(k.P));
   const size_t o_pose0 = L.add<double>(kPS * size_t(k.K)), o_pose1 = L.add<double>(kPS * size_t(k.K));
@@ -675,6 +697,9 @@ int sba_imu_solve(sba_handle* h, const sba_imu_calibration* calib, const sba_imu
   w.blk_jk = reinterpret_cast<int32_t*>(at(o_blk_jk));
   w.blk_tri = reinterpret_cast<int32_t*>(at(o_blk_tri));
   w.tri = reinterpret_cast<int2*>(at(o_tri));
+  w.nslots = int32_t(k.slot_blk.size());
+  w.blk_slot = reinterpret_cast<int32_t*>(at(o_blk_slot));
+  w.slot_blk = reinterpret_cast<int32_t*>(at(o_slot_blk));
   Preint* dpre = reinterpret_cast<Preint*>(at(o_pre));
   w.pre = dpre;
   w.pts[0] = reinterpret_cast<double*>(at(o_pts0));
@@ -728,6 +753,8 @@ int sba_imu_solve(sba_handle* h, const sba_imu_calibration* calib, const sba_imu
       {o_blk_jk, {k.blk_jk.data(), k.blk_jk.size() * 4}},
       {o_blk_tri, {k.blk_tri.data(), k.blk_tri.size() * 4}},
       {o_tri, {k.tri.data(), k.tri.size() * sizeof(int2)}},
+      {o_blk_slot, {k.blk_slot.data(), k.blk_slot.size() * 4}},
+      {o_slot_blk, {k.slot_blk.data(), k.slot_blk.size() * 4}},
       {o_pre, {hpre.data(), hpre.size() * sizeof(Preint)}},
       {o_pts0, {k.pts.data(), k.pts.size() * 8}},
       {o_pts1, {k.pts.data(), k.pts.size() * 8}},

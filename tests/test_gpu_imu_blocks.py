@@ -1,5 +1,8 @@
 """Inertial SBA (sba_imu_solve) in the corners of its kernels, against the FP64 oracle with the bounds of the parity
-scenes: both compute in FP64."""
+scenes: both compute in FP64. The reduced system's factor keeps its nonzero 16 x 16 tiles in shared memory up to 64 of
+them (10 free key frames that share points: 55 tiles; 11: 66; 32 on two-frame tracks: 63; 33: 65), the point kernels
+take 8 lanes per point (up to 13 pairs and 26 observations of a point here), and the pose blocks 512 observations at a
+time."""
 import os
 import sys
 
@@ -24,6 +27,17 @@ def test_information_that_is_not_symmetric(iterations):
     p.observation_infos = np.array(p.observation_infos)
     p.observation_infos[:, 0, 1] = 0.2 * p.observation_infos[:, 0, 0]
     p.observation_infos[:, 1, 0] = 0.1 * p.observation_infos[:, 0, 0]
+    ref = IO.solve(p, calib)
+    q = p.copy()
+    assert imu.IMUBundlerGpuFixedVel(IC.calibration()).solve(q)
+    check_parity(q, ref)
+
+
+# (key frames, fixed, points, track length)
+@pytest.mark.parametrize("shape", [(2, 1, 40, 2), (3, 1, 513, 3), (9, 2, 120, 7), (10, 2, 120, 8), (11, 2, 120, 9),
+                                   (12, 2, 60, 12), (13, 2, 60, 13), (34, 2, 340, 2), (35, 2, 350, 2)])
+def test_route_edges_match_oracle(shape):
+    p, calib, _ = IC.make_scenario(5, shape=shape)
     ref = IO.solve(p, calib)
     q = p.copy()
     assert imu.IMUBundlerGpuFixedVel(IC.calibration()).solve(q)
