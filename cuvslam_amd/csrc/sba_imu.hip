@@ -7,13 +7,13 @@
 //                     and translation columns of W are non-zero), each block summed over its co-observing points in a
 //                     fixed order, and the reduced right-hand side
 //   k_imu_factor      dense Cholesky of S and the two triangular solves in one workgroup (k_imu_factor_lds: tiles in LDS)
-//   k_imu_backsub     dp = Vinv (e_b - sum_j W_ij dc_j), trial points, the points' share of the prediction
-//   k_imu_pose_trial  trial key frames: R Exp(dr), t + R dt, v + dv, biases + db (imu_sba_fixed_vel.cpp:224-240)
-//   k_imu_pose_pred   dc^T (U + 2 lambda diag U) dc by rows
+//   k_imu_apply       dp = Vinv (e_b - sum_j W_ij dc_j), trial points, the points' share of the prediction; trial key
+//                     frames: R Exp(dr), t + R dt, v + dv, biases + db (imu_sba_fixed_vel.cpp:224-240); dc^T (U + 2
+//                     lambda diag U) dc by rows
 //   k_imu_cost        the trial cost: Huber reprojection terms, inertial and random-walk terms, bias prior
 //   k_imu_reduce      the iteration's scalars, summed in a fixed order (deterministic)
-// and after an accepted step k_imu_accept, then the model (k_imu_obs_model, k_imu_edge_model) and the full system
-// (k_imu_point_full, k_imu_pose_full) of the new state (imu_sba_fixed_vel.cpp:455-1004).
+// and after an accepted step k_imu_accept, then the model (k_imu_model: observations and edges) and the full system
+// (k_imu_full: points and key frames) of the new state (imu_sba_fixed_vel.cpp:455-1004).
 #include <hip/hip_runtime.h>
 
 #include <math.h>
@@ -227,9 +227,7 @@ __device__ __forceinline__ bool edge_active(const Window& w, int i) { return !(i
 
 // Residual, Huber weight and Jacobians of every observation at the current state (imu_sba_fixed_vel.cpp:499-566):
 // JR = M [p_imu]x, Jt = -M, Jp = M R^T with M = dproj R_cam_from_imu.
-__global__ __launch_bounds__(kThreads) void k_imu_obs_model(Window w) {
-  const int o = blockIdx.x * blockDim.x + threadIdx.x;
-  if (o >= w.N) return;
+__device__ __forceinline__ void obs_model(const Window& w, int o) {
   ObsModel m{};
   double pi[3], pc[3];
   if (project(w, 0, o, pi, pc)) {
@@ -268,10 +266,10 @@ __global__ __launch_bounds__(kThreads) void k_imu_obs_model(Window w) {
 // Lambda) r, each entry a fixed-order sum.
 __device__ void edge_model_eval(const Window& w, int i, EdgeModel& m);
 
-__global__ __launch_bounds__(kEdgeThreads) void k_imu_edge_model(Window w) {
+__device__ __forceinline__ void edge_model(const Window& w, int i) {
   __shared__ double Js[9][24], LJ[9][25];  // column 24 of LJ: pen Lambda r
   __shared__ double info[81];
-  const int i = blockIdx.x, tid = threadIdx.x;
+  const int tid = threadIdx.x;
   EdgeModel& m = w.em[i];
   const bool active = edge_active(w, i);
   if (!active) {
@@ -300,6 +298,19 @@ __global__ __launch_bounds__(kEdgeThreads) void k_imu_edge_model(Window w) {
     else
       m.g[a] = s;
   }
+}
+
+// The model of the current state: workgroups 0 .. K-2 the inertial edges, the others kThreads observations each. The two
+// do not depend on each other, and an edge is one thread's long chain: in one launch the observations run beside it
+// (10 key frames: 16.0 + 5.3 us in two launches, 14.9 in one; 20 key frames: 17.6 + 7.5, 17.6).
+__global__ __launch_bounds__(kThreads) void k_imu_model(Window w) {
+  const int edges = w.K > 1 ? w.K - 1 : 0;
+  if (blockIdx.x < edges) {  // workgroup-uniform
+    edge_model(w, blockIdx.x);
+    return;
+  }
+  const int o = (blockIdx.x - edges) * kThreads + threadIdx.x;
+  if (o < w.N) obs_model(w, o);
 }
 
 __device__ void edge_model_eval(const Window& w, int i, EdgeModel& m) {
@@ -373,8 +384,8 @@ __device__ __forceinline__ double point_sum(double x) {
 // added by a fixed butterfly; then lane s forms the pairs s, s + kPointLanes, ..., each over its observations in order. A
 // dependent chain of loads (index, then model) per observation bounds it, so the lanes take it side by side: 800 points
 // on 4-frame tracks of two cameras 25.5 -> 6.2 us.
-__global__ __launch_bounds__(kThreads) void k_imu_point_full(Window w) {
-  const int i = (blockIdx.x * kThreads + threadIdx.x) / kPointLanes, s = threadIdx.x % kPointLanes;
+__device__ __forceinline__ void point_full(const Window& w, int t) {
+  const int i = t / kPointLanes, s = t % kPointLanes;
   if (i >= w.P) return;  // whole groups of lanes
   double V[9] = {}, eb[3] = {};
   for (int q = w.point_obs[i] + s; q < w.point_obs[i + 1]; q += kPointLanes) {
@@ -424,15 +435,14 @@ __global__ __launch_bounds__(kThreads) void k_imu_point_full(Window w) {
 // (imu_sba_fixed_vel.cpp:701-1003 with the GPU bundler's penalties, sba_imu_v1.cu:1521-1805). Every element is
 // written by one thread: no atomics, no separate clearing. The reprojection sums: each thread forms all 42 values (the
 // 6 x 6 block, which an information matrix that is not symmetric leaves so, and 6 of the right-hand side) of its
-// observations in registers, a wavefront adds its lanes and the
-// wavefronts are added in order; the edge terms are the H and g blocks that k_imu_edge_model formed. One value per thread
-// over strided slices of the observations read every model 42 times in chains of dependent loads: 20 key frames, 5900
-// points, 76.5 -> 18.2 us; 10 key frames, 800 points, 53.7 -> 16.5.
-__global__ __launch_bounds__(kPoseFullThreads) void k_imu_pose_full(Window w) {
+// observations in registers, a wavefront adds its lanes and the wavefronts are added in order; the edge terms are the
+// H and g blocks of k_imu_model. One value per thread over strided slices of the observations read every model 42 times
+// in chains of dependent loads: 20 key frames, 5900 points, 76.5 -> 18.2 us; 10 key frames, 800 points, 53.7 -> 16.5.
+__device__ __forceinline__ void pose_full(const Window& w, int j) {
   constexpr int kWaves = kPoseFullThreads / 64;
   __shared__ double part[42 * kWaves];
   __shared__ double vis[42];  // the reprojection block (6 x 6) and right-hand side (6)
-  const int j = blockIdx.x, k = w.F + j, tid = threadIdx.x;
+  const int k = w.F + j, tid = threadIdx.x;
   const int n15 = 15 * w.n;
   double val[42] = {};
   for (int q = w.pose_obs[j] + tid; q < w.pose_obs[j + 1]; q += kPoseFullThreads) {
@@ -522,6 +532,16 @@ __global__ __launch_bounds__(kPoseFullThreads) void k_imu_pose_full(Window w) {
     }
     w.ea[15 * j + a] = v;
   }
+}
+
+// The full system of the current state: workgroups 0 .. n-1 the free key frames, the others kPoseFullThreads /
+// kPointLanes points each. Both read the model only, so one launch runs the points beside the key frames (10 key
+// frames: 16.5 + 6.2 us in two launches, 16.3 in one; 20 key frames: 18.2 + 6.5, 18.8).
+__global__ __launch_bounds__(kPoseFullThreads) void k_imu_full(Window w) {
+  if (blockIdx.x < w.n)  // workgroup-uniform
+    pose_full(w, blockIdx.x);
+  else
+    point_full(w, (blockIdx.x - w.n) * kPoseFullThreads + threadIdx.x);
 }
 
 // ---- reduced system ------------------------------------------------------------------------------------------------
@@ -944,9 +964,7 @@ __global__ __launch_bounds__(kFactorThreads) void k_imu_factor_lds(Window w) {
 
 // dp = Vinv (e_b - sum_j W_ij dc_j), the trial point, and the point's share of the prediction
 // dp^T (V + 2 lambda diag V) dp + 2 dp^T sum_j W_ij dc_j (sba_imu_v1.cu:372-394, 767-819).
-__global__ __launch_bounds__(kThreads) void k_imu_backsub(Window w) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= w.P || !*w.chol_ok) return;
+__device__ __forceinline__ void backsub(const Window& w, int i) {
   double t[3] = {0, 0, 0};
   for (int p = w.point_pair[i]; p < w.point_pair[i + 1]; ++p) {
     const double* Wp = w.W + 18 * p;
@@ -975,9 +993,7 @@ __global__ __launch_bounds__(kThreads) void k_imu_backsub(Window w) {
 }
 
 // Trial key frames: R Exp(dr), t + R dt, v + dv, biases + db (imu_sba_fixed_vel.cpp:224-240).
-__global__ __launch_bounds__(64) void k_imu_pose_trial(Window w) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= w.n || !*w.chol_ok) return;
+__device__ __forceinline__ void pose_trial(const Window& w, int j) {
   const int k = w.F + j;
   const double* d = w.rhs + 15 * j;
   const double* X = w.pose[0] + kPS * k;
@@ -998,11 +1014,10 @@ __global__ __launch_bounds__(64) void k_imu_pose_trial(Window w) {
 // Row r of dc^T (U + 2 lambda diag U) dc (sba_imu_v1.cu:821-852), one wavefront per row. U couples a key frame only
 // with its neighbours (the inertial edges), so row r is summed over the column blocks of key frames j-1..j+1, which
 // hold every non-zero of the row (at most 45 columns, one per lane); the lanes are added by a fixed shuffle tree.
-__global__ __launch_bounds__(kThreads) void k_imu_pose_pred(Window w) {
+__device__ __forceinline__ void pose_pred(const Window& w, int r) {
   const int lane = threadIdx.x & 63;
-  const int r = blockIdx.x * (kThreads / 64) + threadIdx.x / 64;
   const int M = 15 * w.n;
-  if (r >= M || !*w.chol_ok) return;  // wavefront-uniform
+  if (r >= M) return;  // wavefront-uniform
   const int jb = r / 15;
   const int c0 = jb > 0 ? 15 * (jb - 1) : 0, c1 = min(M, 15 * (jb + 2));
   const int c = c0 + lane;
@@ -1011,6 +1026,23 @@ __global__ __launch_bounds__(kThreads) void k_imu_pose_pred(Window w) {
   if (c < c1) s = w.U[static_cast<int64_t>(r) * M + c] * dc[c] * (c == r ? 1.0 + 2.0 * w.lambda : 1.0);
   for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off);
   if (lane == 0) w.cpred[r] = dc[r] * s;
+}
+
+// Everything that follows from the step dc: workgroup 0 the trial key frames (kMaxFree at most, a thread each), the next
+// `rows` workgroups the prediction's rows, the others kThreads points each. None reads what another writes, so one launch
+// holds them (20 key frames: 5.9 + 4.6 + 4.6 us and two gaps in three launches, 6.3 in one).
+__global__ __launch_bounds__(kThreads) void k_imu_apply(Window w, int rows) {
+  static_assert(kMaxFree <= kThreads, "the trial key frames are one workgroup's");
+  if (!*w.chol_ok) return;
+  const int b = blockIdx.x, tid = threadIdx.x;
+  if (b == 0) {
+    if (tid < w.n) pose_trial(w, tid);
+  } else if (b <= rows) {
+    pose_pred(w, (b - 1) * (kThreads / 64) + tid / 64);
+  } else {
+    const int i = (b - 1 - rows) * kThreads + tid;
+    if (i < w.P) backsub(w, i);
+  }
 }
 
 // ---- cost ----------------------------------------------------------------------------------------------------------
@@ -1126,10 +1158,10 @@ namespace sba_imu_dev {
 static inline unsigned blocks(int n, int t) { return static_cast<unsigned>((n + t - 1) / t); }
 
 hipError_t imu_model(const Window& w, hipStream_t s) {
-  if (w.N > 0) hipLaunchKernelGGL(k_imu_obs_model, dim3(blocks(w.N, kThreads)), dim3(kThreads), 0, s, w);
-  if (w.K > 1) hipLaunchKernelGGL(k_imu_edge_model, dim3(w.K - 1), dim3(kEdgeThreads), 0, s, w);
-  if (w.P > 0) hipLaunchKernelGGL(k_imu_point_full, dim3(blocks(w.P, kThreads / kPointLanes)), dim3(kThreads), 0, s, w);
-  if (w.n > 0) hipLaunchKernelGGL(k_imu_pose_full, dim3(w.n), dim3(kPoseFullThreads), 0, s, w);
+  const unsigned edges = w.K > 1 ? w.K - 1 : 0, pts = w.P > 0 ? blocks(w.P, kPoseFullThreads / kPointLanes) : 0;
+  if (edges + blocks(w.N, kThreads) > 0)
+    hipLaunchKernelGGL(k_imu_model, dim3(edges + blocks(w.N, kThreads)), dim3(kThreads), 0, s, w);
+  if (w.n + pts > 0) hipLaunchKernelGGL(k_imu_full, dim3(w.n + pts), dim3(kPoseFullThreads), 0, s, w);
   return hipGetLastError();
 }
 
@@ -1142,11 +1174,8 @@ hipError_t imu_step(const Window& w, hipStream_t s) {
     hipLaunchKernelGGL(k_imu_factor_lds, dim3(1), dim3(kFactorThreads), 0, s, w);
   else
     hipLaunchKernelGGL(k_imu_factor, dim3(1), dim3(kFactorThreads), 0, s, w);
-  if (w.P > 0) hipLaunchKernelGGL(k_imu_backsub, dim3(blocks(w.P, kThreads)), dim3(kThreads), 0, s, w);
-  if (w.n > 0) {
-    hipLaunchKernelGGL(k_imu_pose_trial, dim3(blocks(w.n, 64)), dim3(64), 0, s, w);
-    hipLaunchKernelGGL(k_imu_pose_pred, dim3(blocks(15 * w.n, kThreads / 64)), dim3(kThreads), 0, s, w);
-  }
+  const unsigned rows = blocks(15 * w.n, kThreads / 64);
+  hipLaunchKernelGGL(k_imu_apply, dim3(1 + rows + blocks(w.P, kThreads)), dim3(kThreads), 0, s, w, static_cast<int>(rows));
   hipLaunchKernelGGL(k_imu_cost, dim3(blocks(w.N + w.K, kThreads)), dim3(kThreads), 0, s, w, 1);
   hipLaunchKernelGGL(k_imu_reduce, dim3(1), dim3(1024), 0, s, w, 1);
   return hipGetLastError();

@@ -19,7 +19,6 @@
 namespace sba_imu_dev {
 
 constexpr int kThreads = 256;
-constexpr int kEdgeThreads = 256;  // one workgroup per inertial edge
 constexpr int kReducedThreads = 1024, kReducedSlices = 28;  // 36 x 28 partial sums per reduced block
 constexpr int kPoseFullThreads = 512;  // a thread per observation of a key frame
 constexpr int kPointLanes = 8;         // lanes per point of the point kernels
