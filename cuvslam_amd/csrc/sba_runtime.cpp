@@ -37,11 +37,6 @@ hipError_t launch_schur(const Batch& b, hipStream_t s);
 hipError_t launch_reduce(const Batch& b, hipStream_t s);
 hipError_t launch_factor(const Batch& b, double* dbg_S, hipStream_t s, double* store_L = nullptr);
 hipError_t launch_adj_state(const Batch& b, double* spts, double* sposes, const double* a, int op, hipStream_t s);
-hipError_t launch_adj_assemble(const Batch& b, const AdjData& A, bool hess, hipStream_t s);
-hipError_t launch_adj_start(const Batch& b, const AdjData& A, hipStream_t s);
-hipError_t launch_adj_iteration(const Batch& b, AdjData A, int it, hipStream_t s);
-hipError_t launch_adj_obs_grad(const Batch& b, const AdjData& A, const int32_t* orig, hipStream_t s);
-hipError_t launch_adj_inverse(const double* Lst, int n, double* Linv, double* sinv, hipStream_t s);
 hipError_t launch_backsub(const Batch& b, bool initial, hipStream_t s);
 hipError_t launch_large_factor(const Batch& b, int w, int n, hipStream_t s);
 hipError_t launch_winsorize_select(const Batch& b, int w, int np, int kf, double* err, int32_t* pt_of,
@@ -52,6 +47,15 @@ hipError_t launch_gather(const Batch& b, hipStream_t s);
 hipError_t launch_copy_calibrate(float4* dst, const float4* src, int64_t n, hipStream_t s);
 hipError_t launch_mfma_layout(const float* A, const float* B, float* D, hipStream_t s);
 hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t s);
+// The passes of the implicit differentiation are weak references: the runtime also links without them (into the CPU
+// tests, whose stand-ins cover the solve's launches only), and sba_batch_refine and sba_batch_adjoint then return
+// SBA_E_DEVICE.
+#define SBA_WEAK __attribute__((weak))
+SBA_WEAK hipError_t launch_adj_assemble(const Batch& b, const AdjData& A, bool hess, hipStream_t s);
+SBA_WEAK hipError_t launch_adj_start(const Batch& b, const AdjData& A, hipStream_t s);
+SBA_WEAK hipError_t launch_adj_iteration(const Batch& b, AdjData A, int it, hipStream_t s);
+SBA_WEAK hipError_t launch_adj_obs_grad(const Batch& b, const AdjData& A, const int32_t* orig, hipStream_t s);
+SBA_WEAK hipError_t launch_adj_inverse(const double* Lst, int n, double* Linv, double* sinv, hipStream_t s);
 int scratch_setup(int device, void** ptr, size_t* bytes);
 hipError_t set_kernel_attributes();
 }  // namespace sba_dev
@@ -1792,6 +1796,8 @@ int adj_workspace(sba_handle* h, sba_batch* b, AdjData& A) {
 // Factors the Gauss-Newton system of the solution of window 0 (lambda = 0) once and copies its state to FP64.
 // The batch's LM state is left as it was.
 int adj_prepare(sba_handle* h, sba_batch* b, AdjData& A) {
+  if (!launch_adj_assemble || !launch_adj_start || !launch_adj_iteration || !launch_adj_obs_grad || !launch_adj_inverse)
+    return fail(h, SBA_E_DEVICE, "the implicit differentiation's kernels are not linked");
   if (b->win[0].mapped)
     return fail(h, SBA_E_CAPACITY, "implicit differentiation supports windows of at most 40 free key frames");
   int rc = adj_workspace(h, b, A);

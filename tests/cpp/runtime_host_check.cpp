@@ -17,7 +17,6 @@
 #include <string>
 #include <vector>
 
-#include "../../cuvslam_amd/csrc/sba_adjoint.h"
 #include "../../cuvslam_amd/csrc/sba_device.h"
 #include "../../cuvslam_amd/csrc/sba_imu_device.h"
 #include "../../include/cuvslam_sba.h"
@@ -321,12 +320,13 @@ hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t) {
   std::memset(p, 0, bytes);
   return hipSuccess;
 }
+hipError_t launch_adj_obs(const Batch&, int, const double*, const double*, const double*, double*, double*, const double*,
+                          double*, double*, const int32_t*, int32_t*, hipStream_t) { return hipSuccess; }
 hipError_t launch_adj_state(const Batch&, double*, double*, const double*, int, hipStream_t) { return hipSuccess; }
-hipError_t launch_adj_assemble(const Batch&, const AdjData&, bool, hipStream_t) { return hipSuccess; }
-hipError_t launch_adj_start(const Batch&, const AdjData&, hipStream_t) { return hipSuccess; }
-hipError_t launch_adj_iteration(const Batch&, AdjData, int, hipStream_t) { return hipSuccess; }
-hipError_t launch_adj_obs_grad(const Batch&, const AdjData&, const int32_t*, hipStream_t) { return hipSuccess; }
-hipError_t launch_adj_inverse(const double*, int, double*, double*, hipStream_t) { return hipSuccess; }
+hipError_t launch_adj_chol(const double*, int, const double*, double*, const int32_t*, hipStream_t) { return hipSuccess; }
+hipError_t launch_adj_linv(const double*, int, double*, hipStream_t) { return hipSuccess; }
+hipError_t launch_adj_vec(const Batch&, double*, double*, double*, double*, double*, double*, double*, double*, double*,
+                          double*, int32_t*, double, int, int, int, hipStream_t) { return hipSuccess; }
 hipError_t launch_winsorize_select(const Batch&, int, int, int, double*, int32_t*, int32_t*, uint8_t*, int32_t*, hipStream_t) {
   return hipSuccess;
 }
