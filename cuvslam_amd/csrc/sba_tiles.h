@@ -57,27 +57,50 @@ __device__ __forceinline__ double sum_row16(double x) {  // over the 16 lanes of
   return x;
 }
 
-// An estimate e of 1/sqrt(d) refined by a third-order step (the series of (1 - h)^-1/2 with h = 1 - d e^2: the cube of
-// the hardware estimate's error is below rounding, its square is not always), and 1/sqrt(d) from that estimate.
-__device__ __forceinline__ double refine_rsqrt(double d, double e) {
-  const double h = 1.0 - d * e * e;
+// 1/sqrt(d) of a normal positive d: the hardware estimate e refined by a third-order step (the series of (1 - h)^-1/2
+// with h = 1 - d e^2: the cube of the estimate's error is below rounding, its square is not always). Not a number for
+// every other d, zero and infinity included.
+__device__ __forceinline__ double rsqrt1(double d) {
+  const double e = __builtin_amdgcn_rsq(d), h = 1.0 - d * e * e;
   return e + e * h * (0.5 + 0.375 * h);
 }
-__device__ __forceinline__ double rsqrt1(double d) { return refine_rsqrt(d, __builtin_amdgcn_rsq(d)); }
+
+// r[k] = x of the lane of the same column (lane % 16) in row k (lanes 16 k .. 16 k + 15), in every lane.
+__device__ __forceinline__ void rows_of(double x, double (&r)[4]) {
+  auto half = [](unsigned w, unsigned (&o)[4]) {
+    const auto a = __builtin_amdgcn_permlane32_swap(w, w, false, false);      // rows 0 1 0 1 and 2 3 2 3
+    const auto b = __builtin_amdgcn_permlane16_swap(a[0], a[0], false, false);
+    const auto c = __builtin_amdgcn_permlane16_swap(a[1], a[1], false, false);
+    o[0] = b[0];
+    o[1] = b[1];
+    o[2] = c[0];
+    o[3] = c[1];
+  };
+  unsigned lo[4], hi[4];
+  half(__double2loint(x), lo);
+  half(__double2hiint(x), hi);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) r[k] = __hiloint2double(hi[k], lo[k]);
+}
 
 // Cholesky A = U^T U of a symmetric 16 x 16 tile held by one wavefront in the FP64 matrix-core layout (cell
 // (4v + lane/16, lane%16) in t[v]) together with X = U^-T, as one elimination of [A | I] by panels of four rows.
-// Register v of the layout is exactly the panel of rows 4v..4v+3, and it is at once the B operand of a 4 x 16 factor
-// and the A operand of its transpose, so a panel step needs no data movement:
-//   the 4 x 4 diagonal block is broadcast with readlane, factored and inverted by every lane (M = L_vv^-1);
-//   U_v = M A_v and X_v = M I_v, one matrix instruction each; A -= U_v^T U_v and I -= U_v^T X_v, one each.
+// Register v of the layout is exactly the panel of rows 4v..4v+3:
+//   the 4 x 4 diagonal block is broadcast with readlane and factored by every lane (the plain recurrence, L_vv);
+//   U_v = L_vv^-1 A_v and X_v = L_vv^-1 I_v by forward substitution, every lane with its column's four rows;
+//   A -= U_v^T U_v and I -= U_v^T X_v, one matrix instruction each: the panel is at once the B operand and the A operand
+//   of its transpose.
 // On return t holds U (zero below the diagonal), X^T is written to xt (row-major) and 1 / U_ii to rdiag. False on a
-// non-positive pivot (the values are then dropped by the callers).
+// pivot that is not positive and finite (the values are then dropped by the callers).
 //
-// A serial chain bounds it: four 4 x 4 factors (a reciprocal square root and a few dependent FMAs per pivot) and two
-// dependent matrix instructions each. Measured alone on one wavefront: 2.67 us with a column-by-column factorization
-// and a forward substitution for X through LDS, 1.90 us as a column-by-column elimination of [A | I], 1.72 us in this
-// form; the reconstruction error of a random tile fell from 9e-16 to 7e-16, that of X from 8e-16 to 3e-16.
+// A serial chain bounds it: 16 reciprocal square roots with a few dependent FMAs each, and one matrix instruction per
+// panel between them; the substitutions run beside the chain of their own block. Measured alone on one wavefront: 1.07 us;
+// 1.32 us with the rows as products with the explicit inverse of L_vv and every second square root started from a 2 x 2
+// determinant; 1.80 us as a column-by-column factorization with X formed through LDS. Backward stable: over 2000 tiles
+// each with second pivots of a relative size of 1 to 1e-15, |U^T U - A| stays within 9e-16 of sqrt(a_ii a_jj) and
+// |U^T X - I| within 3.3e-16 of |U^T| |X| (6e-15 and 8e-15 column by column; with the explicit inverse both grew with
+// the block's condition, to 1e-10 and 1e-4 at 1e-12, and a determinant that cancelled to zero gave infinities that
+// passed as a good factor).
 __device__ inline bool factor_tile(double4v& t, double* xt, double* rdiag, int lane) {
   const int row = lane >> 4, col = lane & 15;
   double4v x, u;
@@ -90,38 +113,27 @@ __device__ inline bool factor_tile(double4v& t, double* xt, double* rdiag, int l
     auto at = [&](int r, int c) { return readlane_d(t[v], 16 * r + 4 * v + c); };
     const double a00 = at(0, 0), a01 = at(0, 1), a11 = at(1, 1), a02 = at(0, 2), a12 = at(1, 2), a03 = at(0, 3),
                  a13 = at(1, 3), a22 = at(2, 2), a23 = at(2, 3), a33 = at(3, 3);
-    // Pivots in pairs: the second of a pair is det / first, so the estimates of both reciprocal square roots start
-    // together; the second is then refined against the pivot itself, which keeps the accuracy of the plain recurrence.
-    const double i0 = rsqrt1(a00), f1 = __builtin_amdgcn_rsq(a00 * a11 - a01 * a01) * a00;
-    const double l10 = a01 * i0, l20 = a02 * i0, l30 = a03 * i0;
-    const double d1 = a11 - l10 * l10, i1 = refine_rsqrt(d1, f1 * i0);
+    const double i0 = rsqrt1(a00), l10 = a01 * i0, l20 = a02 * i0, l30 = a03 * i0;
+    const double i1 = rsqrt1(a11 - l10 * l10);
     const double l21 = (a12 - l10 * l20) * i1, l31 = (a13 - l10 * l30) * i1;
-    const double d2 = (a22 - l20 * l20) - l21 * l21, b23 = (a23 - l20 * l30) - l21 * l31,
-                 b33 = (a33 - l30 * l30) - l31 * l31;
-    const double i2 = rsqrt1(d2), f3 = __builtin_amdgcn_rsq(d2 * b33 - b23 * b23) * d2;
-    const double l32 = b23 * i2;
-    const double d3 = b33 - l32 * l32, i3 = refine_rsqrt(d3, f3 * i2);
-    ok = ok && a00 > 0.0 && d1 > 0.0 && d2 > 0.0 && d3 > 0.0;
-    // M = L_vv^-1 as the A operand: lane l holds M[l % 16][l / 16], rows past the fourth zero
-    const double m10 = -(l10 * i0) * i1;
-    const double q20 = l20 * i0 + l21 * m10, q21 = l21 * i1, q30 = l30 * i0 + l31 * m10, q31 = l31 * i1;
-    const double m20 = -q20 * i2, m21 = -q21 * i2;
-    double m = lane == 0 ? i0 : 0.0;
-    m = lane == 1 ? m10 : m;
-    m = lane == 17 ? i1 : m;
-    m = lane == 2 ? m20 : m;
-    m = lane == 18 ? m21 : m;
-    m = lane == 34 ? i2 : m;
-    m = lane == 35 ? -(l32 * i2) * i3 : m;
-    m = lane == 3 ? -(q30 + l32 * m20) * i3 : m;
-    m = lane == 19 ? -(q31 + l32 * m21) * i3 : m;
-    m = lane == 51 ? i3 : m;
-    const double4v zero = {0.0, 0.0, 0.0, 0.0};
-    const double uv = mfma64(m, t[v], zero)[0];
+    const double i2 = rsqrt1((a22 - l20 * l20) - l21 * l21);
+    const double l32 = ((a23 - l20 * l30) - l21 * l31) * i2;
+    const double i3 = rsqrt1(((a33 - l30 * l30) - l31 * l31) - l32 * l32);
+    ok = ok && i0 > 0.0 && i1 > 0.0 && i2 > 0.0 && i3 > 0.0;
+    auto solve = [&](double b) {  // this lane's entry of L_vv^-1 b
+      double r[4];
+      rows_of(b, r);
+      r[0] *= i0;
+      r[1] = (r[1] - l10 * r[0]) * i1;
+      r[2] = ((r[2] - l20 * r[0]) - l21 * r[1]) * i2;
+      r[3] = (((r[3] - l30 * r[0]) - l31 * r[1]) - l32 * r[2]) * i3;
+      return row < 2 ? (row == 0 ? r[0] : r[1]) : (row == 2 ? r[2] : r[3]);
+    };
+    const double uv = solve(t[v]);
     // The next panel waits for A only, so its product goes first. Rows up to this panel are final in u and x and
     // columns up to it are eliminated: what the products leave there is not read again.
     if (v < 3) t = mfma64(-uv, uv, t);
-    const double xv = mfma64(m, x[v], zero)[0];
+    const double xv = solve(x[v]);
     if (v < 3) {
       const double4v xn = mfma64(-uv, xv, x);
 #pragma unroll

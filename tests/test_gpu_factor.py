@@ -1,5 +1,8 @@
 """The 16 x 16 diagonal factor of the reduced camera system at the places where its four-row panels can go wrong: a
-non-positive pivot at every row of a tile, and rows of very different scale."""
+non-positive pivot at every row of a tile, rows of very different scale, and pivots that nearly cancel."""
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -47,3 +50,22 @@ def test_rows_of_different_scale(solver, n, decades):
     H = A * s[:, None] * s[None, :]
     y, ref = x / s, np.linalg.solve(H, b * s)
     assert np.linalg.norm(y - ref) <= 8 * n * (n + 1) * np.finfo(float).eps * np.linalg.cond(H) * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("n, row", [(12, 0), (12, 2), (24, 22), (48, 44), (48, 46), (96, 94)])
+@pytest.mark.parametrize("a", [2.0, 3.0, 7.0, 11.0, 13.0])
+def test_a_singular_pair_fails_or_stays_finite(solver, n, row, a):
+    # the second pivot of the pair is zero but for rounding; (48, 46) and (96, 94) end in the last pivot of the last tile,
+    # which no later pivot checks
+    A = np.eye(n)
+    A[row:row + 2, row:row + 2] = a
+    x, rc = solver.debug_factor(A, np.ones(n))
+    assert rc == ca.sba._lib.SBA_E_INFEASIBLE or np.isfinite(x).all()
+
+
+
+def test_tile_factor_is_backward_stable():
+    # the factor and inverse themselves: a solve shows their errors only through the condition of the system
+    r = subprocess.run([os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "factor_tile_check")], text=True,
+                       capture_output=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
