@@ -943,9 +943,10 @@ __global__ __launch_bounds__(kFactorThreads) void k_factor(Batch b, double* dbg_
     // wavefront 0: the diagonal factors
     __syncthreads();
     // 2. factorization; K = -1 only factors tile (0, 0). The other wavefronts run their own copy of the loop
-    //    with the same barriers.
+    //    with the same barriers. The flag is not read at K = -1: no barrier lies between that read and the write of a
+    //    failed tile (0, 0).
     for (int K = -1; K + 1 < T; ++K) {
-      if (flag) break;
+      if (K >= 0 && flag) break;
       double* tk = sDg + 256 * (K + 1);
       double4v dt;
 #pragma unroll
@@ -1044,7 +1045,7 @@ __global__ __launch_bounds__(kFactorThreads) void k_factor(Batch b, double* dbg_
     }
     __syncthreads();
     for (int K = -1; K + 1 < T; ++K) {
-      if (flag) break;
+      if (K >= 0 && flag) break;
       if (K >= 0) {
         // panel U_KI = X_KK A_KI (the B operand of chunk q is register q of the tile itself), published to LDS
         const double* xt = sXT + 256 * K;

@@ -206,7 +206,7 @@ __device__ bool factor_block(double* sm, int* flag, double* Xg, double* rhs, int
   };
   if (wave == 0) {
     for (int K = -1; K < T; ++K) {
-      if (*flag) break;
+      if (K >= 0 && *flag) break;  // at K = -1 no barrier lies between the read and a failed tile's write
       if (K >= 0) {
         const double yk = forward(K);
         if (lane < 16) ys[16 * K + lane] = yk;
@@ -236,7 +236,7 @@ __device__ bool factor_block(double* sm, int* flag, double* Xg, double* rhs, int
       inv[s] = double4v{0.0, 0.0, 0.0, 0.0};
     }
     for (int K = -1; K < T; ++K) {
-      if (*flag) break;
+      if (K >= 0 && *flag) break;
       if (K >= 0) {
         const double* xt = sXT + 256 * K;
         const double yk = forward(K);
