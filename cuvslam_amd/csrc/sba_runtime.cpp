@@ -841,7 +841,7 @@ int64_t default_chunk_pairs(int64_t total_pairs, double record_work) {
   constexpr int64_t kResident = 512;
   constexpr double kRecordBytes = 40.0 * 1024 * 1024;
   const int64_t share = std::max<int64_t>(total_pairs / kResident, static_cast<int64_t>(record_work / kRecordBytes));
-  return std::min<int64_t>(std::max<int64_t>(std::min(kCoarseChunkPairs, share), total_pairs / 8192), 65536);
+  return std::min<int64_t>(std::max<int64_t>({1, std::min(kCoarseChunkPairs, share), total_pairs / 8192}), 65536);
 }
 
 // The launch sequence of one solve. With events, each kernel class is timed (eager mode only).
@@ -1921,7 +1921,7 @@ int sba_autotune_chunks(sba_handle* h, const sba_problem_view* problems, int32_t
   HIP_TRY(hipSetDevice(h->opt.device));
   int64_t base = 0;
   {
-    // the default candidates bracket the heuristic: x1/4 .. x4
+    // the default candidates bracket the heuristic
     sba_batch* probe = nullptr;
     const int32_t saved = h->opt.chunk_pairs;
     h->opt.chunk_pairs = 0;
@@ -1933,8 +1933,13 @@ int sba_autotune_chunks(sba_handle* h, const sba_problem_view* problems, int32_t
   }
   std::vector<int32_t> cand(candidates, candidates + n_candidates);
   if (cand.empty()) {
-    for (int64_t c : {base / 4, base / 2, base, 2 * base, 4 * base})
-      cand.push_back(static_cast<int32_t>(std::max<int64_t>(256, c)));
+    // The heuristic itself and x1/4 .. x4, from a full tile's pairs up: a chunk never has less than a tile, so smaller
+    // sizes would time the same plan again (13.9k pairs: the heuristic gives 27, one tile per chunk).
+    const int64_t mid = std::max<int64_t>(base, kTilePairs);
+    for (int64_t c : {base, mid / 4, mid / 2, mid, 2 * mid, 4 * mid}) {
+      const int32_t v = static_cast<int32_t>(c == base ? c : std::max<int64_t>(kTilePairs, c));
+      if (std::find(cand.begin(), cand.end(), v) == cand.end()) cand.push_back(v);
+    }
   }
   const int32_t saved = h->opt.chunk_pairs;
   float best = 0.f;
@@ -2028,7 +2033,9 @@ int sba_autotune_table(sba_handle* h, const char* path, const sba_problem_view* 
   int32_t best_b = best;
   float best_ms = 0.f;
   for (int32_t m : {1, 2, 4, 8}) {
-    h->opt.bchunk_pairs = best * m;
+    // multiples below a full tile would all be one tile per chunk
+    const int32_t bchunk = m == 1 ? best : m * std::max(best, kTilePairs / 2);
+    h->opt.bchunk_pairs = bchunk;
     sba_batch* b = nullptr;
     if ((rc = sba_batch_create(h, problems, n, &b)) != SBA_OK) break;
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -2048,7 +2055,7 @@ int sba_autotune_table(sba_handle* h, const char* path, const sba_problem_view* 
     if (rc != SBA_OK) break;
     if (m == 1 || ms < best_ms) {
       best_ms = ms;
-      best_b = best * m;
+      best_b = bchunk;
     }
   }
   h->opt.chunk_pairs = saved_c;

@@ -145,18 +145,18 @@ int sba_batch_kernel_times(sba_handle* h, sba_batch* b, float* ms_per_class, int
 /* Autotuner of the batched launch's work granularity (pairs per Schur chunk; the back-substitution chunks follow
  * it). Each candidate builds the batch, runs one warm-up solve and times `repeats` solves with HIP events on the
  * handle's stream; the fastest is returned in best_chunk_pairs (set it as sba_options.chunk_pairs of a handle).
- * candidates == NULL or n_candidates == 0 tries the built-in heuristic scaled by 1/4 .. 4; ms_per_candidate
- * [optional, n_candidates] receives the mean time per solve of each given candidate. No reference counterpart
- * (the reference solves one window per call). */
+ * candidates == NULL or n_candidates == 0 tries the built-in heuristic and that scaled by 1/4 .. 4, the scaled ones
+ * from a tile's 256 pairs up; ms_per_candidate [optional, n_candidates] receives the mean time per solve of each
+ * given candidate. No reference counterpart (the reference solves one window per call). */
 int sba_autotune_chunks(sba_handle* h, const sba_problem_view* problems, int32_t n, const int32_t* candidates,
                         int32_t n_candidates, int32_t repeats, int32_t* best_chunk_pairs, float* ms_per_candidate);
 
 /* The autotuner with a table: looks up the batch's shape class (device architecture, loss, window count, total
  * observations to two significant digits, largest free key-frame count) in the text file `path`; when it is not
  * there, tunes the Schur chunk size (sba_autotune_chunks over its default candidates), then the back-substitution
- * chunk size (1, 2, 4 and 8 times the Schur size), and appends the result. *from_table [optional] is 1 when the
- * sizes came from the file. Set the results as sba_options.chunk_pairs and bchunk_pairs of a handle. No reference
- * counterpart. */
+ * chunk size (1, 2, 4 and 8 times the Schur size, the multiples from a tile's 256 pairs up), and appends the result.
+ * *from_table [optional] is 1 when the sizes came from the file. Set the results as sba_options.chunk_pairs and
+ * bchunk_pairs of a handle. No reference counterpart. */
 int sba_autotune_table(sba_handle* h, const char* path, const sba_problem_view* problems, int32_t n, int32_t repeats,
                        int32_t* chunk_pairs, int32_t* bchunk_pairs, int32_t* from_table);
 

@@ -33,3 +33,18 @@ def test_default_chunks_match_one_chunk(points, key_frames):
         assert ca.SchurComplementBundlerGpu(loss=ca.LOSS_STUDENT_T, fixed_iterations=True, chunk_pairs=chunk_pairs).solve(q)
         out.append(q)
     assert abs(out[0].last_cost_f64 - out[1].last_cost_f64) <= 1e-6 * out[1].last_cost_f64
+
+
+@pytest.mark.parametrize("points, key_frames", [(40, 4), (200, 5), (2000, 7)])
+def test_autotuner_times_the_default(points, key_frames, tmp_path):
+    # below a tile per workgroup of the chip the default is one tile per chunk; two tiles per chunk take 1.3 times as long
+    # or more, so the tuner must come back with the default's plan (40 points: the default is the smallest size, one pair)
+    p, _, _ = ca.scene.generate(seed=4, num_points=points, num_keyframes=key_frames, num_fixed_keyframes=2, max_iterations=7)
+    make = lambda **kw: ca.SchurComplementBundlerGpu(loss=ca.LOSS_STUDENT_T, fixed_iterations=True, **kw)  # noqa: E731
+    best, _ = make().autotune([p], repeats=10)
+    default = make().batch([p]).info()["chunks"]
+    assert default > 1 and best > 0 and make(chunk_pairs=best).batch([p]).info()["chunks"] == default
+    table = str(tmp_path / "table.txt")
+    tuned = make().autotune_table([p], table, repeats=10)
+    assert make(chunk_pairs=tuned[0]).batch([p]).info()["chunks"] == default and not tuned[2]
+    assert make().autotune_table([p], table) == (tuned[0], tuned[1], True)  # read back from the file
