@@ -1,5 +1,5 @@
 """Windows cut into few and many chunks: the record reduction at the chunk counts where it changes (sums of eight loads at
-a time, one entry per thread below 24 chunks and four wavefronts per entry from there), and the default chunk size."""
+a time, one entry per thread below 64 chunks and four wavefronts per entry from there), and the default chunk size."""
 import numpy as np
 import pytest
 
@@ -8,7 +8,7 @@ import cuvslam_amd as ca
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("chunks", [1, 2, 7, 8, 9, 16, 23, 24, 25, 31, 33, 40])
+@pytest.mark.parametrize("chunks", [1, 2, 7, 8, 9, 16, 23, 24, 25, 31, 33, 40, 63, 64, 65, 97])
 def test_reduced_system_does_not_depend_on_the_chunk_count(chunks):
     # a Schur tile holds 16 points, so 16 points per tile and one tile per chunk give the wanted count
     p, _, _ = ca.scene.generate(seed=3, num_points=16 * chunks, num_keyframes=8, num_fixed_keyframes=2, z_min=8.0,
