@@ -992,72 +992,23 @@ int host_staging(sba_handle* h, size_t bytes, char** out) {
 
 namespace {
 
-// Packs and plans the windows on the host, takes the batch's device block from `memory`, uploads, and (graph)
-// records the whole solve as one hipGraph. On failure nothing is left allocated by the batch itself.
-int build_batch_impl(sba_handle* h, const sba_problem_view* problems, int32_t n, bool graph, bool wait_upload,
-                     const MemorySource& memory, sba_batch** out) {
-  *out = nullptr;
-  TraceRange tr("sba pack and plan");
-  HostPack& H = h->pack;
-  HIP_TRY(hipStreamSynchronize(h->stream));  // no copy of an earlier batch still reads the packing buffers
-  H.clear();
-  std::unique_ptr<sba_batch, int (*)(sba_batch*)> owned(new (std::nothrow) sba_batch, free_batch);
-  sba_batch* b = owned.get();
-  if (!b) return fail(h, SBA_E_INVALID, "out of host memory");
-  b->n = n;
-  b->win.resize(n);
-  b->status_pre.assign(n, SBA_OK);
-  int64_t sred_off = 0, a_off = 0, dc_off = 0;
-  int max_nc = 1, max_ncam = 1, max_ncf = 1, max_rec = 0;
-  int rc = SBA_OK;
-  if ((rc = pack_windows(h, problems, n, H, b->win)) != SBA_OK) return rc;
-  for (int w = 0; w < n; ++w) {
-    const sba_problem_view& p = problems[w];
-    WindowDesc& W = b->win[w];
-    if (W.np == 0 || W.nc == 0 || W.no == 0) b->status_pre[w] = SBA_E_EMPTY;
-    W.nt = W.mapped ? 0 : (6 * W.ncf + 15) / 16;
-    W.rec = W.mapped ? 0 : 256 * (W.nt * (W.nt + 1) / 2) + 33 * W.ncf;
-    W.sred_off = sred_off;
-    sred_off += W.rec;
-    max_rec = std::max(max_rec, W.rec);
-    W.dc_off = static_cast<int32_t>(dc_off);
-    dc_off += 6 * W.ncf;
-    const int nn = 6 * W.ncf;
-    W.a_off = 0;
-    if (W.mapped) {
-      // FP64 A (n x n), rhs, diag U, the inverses of the diagonal blocks
-      W.a_off = a_off;
-      a_off += static_cast<int64_t>(nn) * nn + 2 * nn + static_cast<int64_t>((nn + 63) / 64) * 64 * 64;
-      b->mapped.push_back(w);
-    }
-    if (b->point_order.size() != static_cast<size_t>(n)) b->point_order.resize(n);
-    b->point_order[w] = H.sorts[w].order;
-    max_nc = std::max(max_nc, W.nc);
-    max_ncam = std::max(max_ncam, W.ncam);
-    max_ncf = std::max(max_ncf, W.ncf);
-    b->max_iter = std::max(b->max_iter, p.max_iterations);
-    // an empty window never runs: the initial decision sees zero observations as infeasible, so mark it here
-    if (b->status_pre[w] != SBA_OK) W.max_iterations = 0;
-  }
-  b->total_obs = static_cast<int64_t>(H.obs_xy.size());
-  b->total_pairs = static_cast<int64_t>(H.pair_pose.size());
-
-  b->pairs0 = H.sorts[0].npairs;
-  b->btiles0 = static_cast<int>(H.wbtiles[0].size());
-  // chunks: consecutive tiles of one window, about chunk_pairs pairs of work each; each owns one record
-  int64_t target = h->opt.chunk_pairs;
-  if (target <= 0) {
-    double record_work = 0.0;
-    for (int w = 0; w < n; ++w) record_work += static_cast<double>(H.sorts[w].npairs) * b->win[w].rec * sizeof(float);
-    target = default_chunk_pairs(b->total_pairs, record_work);
-    b->default_chunk = target;
-  }
-  const int64_t btarget = h->opt.bchunk_pairs > 0 ? h->opt.bchunk_pairs : target;
+// Groups the packed tiles of b's windows into Schur chunks of about `target` pairs and back-substitution chunks of about
+// `btarget`, with the record offsets, the mapped windows' local key frames and gather plan and the reduction's work
+// list. Returns the floats of all records. Can be called again with other sizes.
+int64_t plan_chunks(sba_batch* b, HostPack& H, int64_t target, int64_t btarget) {
+  const int n = b->n;
+  // chunks: consecutive tiles of one window, about chunk_pairs pairs of work each; each owns one record.
   // In a mapped window a chunk also stages at most kMaxFreePoses free key frames: its map lists them in
   // increasing order and its pairs carry their index in that list.
   pinned_vector<Chunk>& chunks = H.chunks;
   pinned_vector<int32_t>& chunk_map = H.chunk_map;
   int64_t part_off = 0;
+  chunks.clear();
+  chunk_map.clear();
+  H.gfirst.clear();
+  H.gcon.clear();
+  H.bchunks.clear();
+  for (WindowDesc& W : b->win) W.nchunks = W.nbchunks = 0;
   {
     size_t t = 0;
     int last_w = -1;
@@ -1188,34 +1139,119 @@ int build_batch_impl(sba_handle* h, const sba_problem_view* problems, int32_t n,
     const int per = W.nchunks < kReduceSplit ? 256 : 64;
     red_first[w + 1] = red_first[w] + (W.mapped ? 0 : (W.rec + per - 1) / per);
   }
+  return part_off;
+}
 
+// The device block of the planned batch: `part`, `sred`, `a` and `dc` elements of records, reduced records, mapped windows'
+// FP64 systems and steps; `pair_streams`: pairs have their own copy of their first observation.
+Layout lay_out(sba_batch* b, const HostPack& H, int64_t part, int64_t sred, int64_t a, int64_t dc, bool pair_streams) {
   Batch& d = b->dev;
-  d.n_windows = n;
-  d.red_blocks = red_first[n];
-  d.n_chunks = static_cast<int32_t>(chunks.size());
-  d.n_bchunks = static_cast<int32_t>(bchunks.size());
-  d.n_points = static_cast<int32_t>(H.pts.size());
-  d.n_poses = static_cast<int32_t>(H.poses.size() / 3);
-  d.n_cams = static_cast<int32_t>(H.cams.size() / 3);
-  d.loss = h->opt.loss;
-  d.fixed_iterations = h->opt.fixed_iterations;
-  d.max_rec = max_rec;
-  d.max_nc = max_nc;
   Layout L;
   L.upload(d.win, b->win);
   L.upload(d.tiles, H.tiles);
-  L.upload(d.chunks, chunks);
-  L.upload(d.chunk_map, chunk_map);
+  L.upload(d.chunks, H.chunks);
+  L.upload(d.chunk_map, H.chunk_map);
   L.upload(d.gfirst, H.gfirst);
   L.upload(d.gcon, H.gcon);
   L.upload(d.btiles, H.btiles);
-  L.upload(d.bchunks, bchunks);
-  L.upload(d.red_first, red_first);
+  L.upload(d.bchunks, H.bchunks);
+  L.upload(d.red_first, H.red_first);
   L.upload(d.obs_xy, H.obs_xy);
   L.upload(d.obs_info, H.obs_info);
   L.upload(d.pair_obs, H.pair_obs);
   L.upload(d.pair_pose, H.pair_pose);
   L.upload(d.pair_rec, H.pair_rec);
+  if (pair_streams) {
+    L.upload(d.pair_xy, H.pair_xy);
+    L.upload(d.pair_info, H.pair_info);
+  }
+  L.upload(d.point_pair, H.point_pair);
+  L.upload(d.point_nfree, H.point_nfree);
+  L.upload(d.pts_init, H.pts);
+  L.upload(d.poses_init, H.poses);
+  L.upload(d.cams, H.cams);
+  L.upload(b->obs_orig, H.obs_orig);
+  L.begin_zeroed();
+  L.zeroed(d.st, static_cast<size_t>(b->n));
+  L.zeroed(d.pts0, H.pts.size());
+  L.zeroed(d.pts1, H.pts.size());
+  L.zeroed(d.paux, 3 * H.pts.size());
+  L.zeroed(d.poses0, H.poses.size());
+  L.zeroed(d.poses1, H.poses.size());
+  L.zeroed(d.part, static_cast<size_t>(part));
+  L.zeroed(d.sred, static_cast<size_t>(sred));
+  L.zeroed(d.A, static_cast<size_t>(a));
+  L.zeroed(d.dc, static_cast<size_t>(dc));
+  L.zeroed(d.dc64, static_cast<size_t>(dc));
+  L.zeroed(d.out_pts, H.pts.size());
+  L.zeroed(d.out_poses, H.poses.size());
+  L.zeroed(d.trace, static_cast<size_t>(b->n) * kTrace);
+  L.zeroed(d.bpart, H.bchunks.size());
+  return L;
+}
+
+// Packs and plans the windows on the host, takes the batch's device block from `memory`, uploads, and (graph)
+// records the whole solve as one hipGraph. On failure nothing is left allocated by the batch itself. Small chunks trade
+// memory for time (a record each): where the default chunk size would need more than `memory_limit` bytes, the chunks
+// are planned again at kCoarseChunkPairs.
+int build_batch_impl(sba_handle* h, const sba_problem_view* problems, int32_t n, bool graph, bool wait_upload,
+                     const MemorySource& memory, size_t memory_limit, sba_batch** out) {
+  *out = nullptr;
+  TraceRange tr("sba pack and plan");
+  HostPack& H = h->pack;
+  HIP_TRY(hipStreamSynchronize(h->stream));  // no copy of an earlier batch still reads the packing buffers
+  H.clear();
+  std::unique_ptr<sba_batch, int (*)(sba_batch*)> owned(new (std::nothrow) sba_batch, free_batch);
+  sba_batch* b = owned.get();
+  if (!b) return fail(h, SBA_E_INVALID, "out of host memory");
+  b->n = n;
+  b->win.resize(n);
+  b->status_pre.assign(n, SBA_OK);
+  int64_t sred_off = 0, a_off = 0, dc_off = 0;
+  int max_nc = 1, max_ncam = 1, max_ncf = 1, max_rec = 0;
+  int rc = SBA_OK;
+  if ((rc = pack_windows(h, problems, n, H, b->win)) != SBA_OK) return rc;
+  for (int w = 0; w < n; ++w) {
+    const sba_problem_view& p = problems[w];
+    WindowDesc& W = b->win[w];
+    if (W.np == 0 || W.nc == 0 || W.no == 0) b->status_pre[w] = SBA_E_EMPTY;
+    W.nt = W.mapped ? 0 : (6 * W.ncf + 15) / 16;
+    W.rec = W.mapped ? 0 : 256 * (W.nt * (W.nt + 1) / 2) + 33 * W.ncf;
+    W.sred_off = sred_off;
+    sred_off += W.rec;
+    max_rec = std::max(max_rec, W.rec);
+    W.dc_off = static_cast<int32_t>(dc_off);
+    dc_off += 6 * W.ncf;
+    const int nn = 6 * W.ncf;
+    W.a_off = 0;
+    if (W.mapped) {
+      // FP64 A (n x n), rhs, diag U, the inverses of the diagonal blocks
+      W.a_off = a_off;
+      a_off += static_cast<int64_t>(nn) * nn + 2 * nn + static_cast<int64_t>((nn + 63) / 64) * 64 * 64;
+      b->mapped.push_back(w);
+    }
+    if (b->point_order.size() != static_cast<size_t>(n)) b->point_order.resize(n);
+    b->point_order[w] = H.sorts[w].order;
+    max_nc = std::max(max_nc, W.nc);
+    max_ncam = std::max(max_ncam, W.ncam);
+    max_ncf = std::max(max_ncf, W.ncf);
+    b->max_iter = std::max(b->max_iter, p.max_iterations);
+    // an empty window never runs: the initial decision sees zero observations as infeasible, so mark it here
+    if (b->status_pre[w] != SBA_OK) W.max_iterations = 0;
+  }
+  b->total_obs = static_cast<int64_t>(H.obs_xy.size());
+  b->total_pairs = static_cast<int64_t>(H.pair_pose.size());
+
+  b->pairs0 = H.sorts[0].npairs;
+  b->btiles0 = static_cast<int>(H.wbtiles[0].size());
+  int64_t target = h->opt.chunk_pairs;
+  const bool use_default = target <= 0;
+  if (use_default) {
+    double record_work = 0.0;
+    for (int w = 0; w < n; ++w) record_work += static_cast<double>(H.sorts[w].npairs) * b->win[w].rec * sizeof(float);
+    target = default_chunk_pairs(b->total_pairs, record_work);
+    b->default_chunk = target;
+  }
   bool copies = false;  // wide points' pair copies
   for (int w = 0; w < n; ++w) copies = copies || H.sorts[w].ndup > 0;
   const bool pair_streams = H.obs_xy.size() != H.pair_rec.size() || copies;
@@ -1227,31 +1263,25 @@ int build_batch_impl(sba_handle* h, const sba_problem_view* problems, int32_t n,
       H.pair_xy[q] = H.obs_xy[H.pair_rec[q].x];
       H.pair_info[q] = H.obs_info[H.pair_rec[q].x];
     }
-    L.upload(d.pair_xy, H.pair_xy);
-    L.upload(d.pair_info, H.pair_info);
   }
-  L.upload(d.point_pair, H.point_pair);
-  L.upload(d.point_nfree, H.point_nfree);
-  L.upload(d.pts_init, H.pts);
-  L.upload(d.poses_init, H.poses);
-  L.upload(d.cams, H.cams);
-  L.upload(b->obs_orig, H.obs_orig);
-  L.begin_zeroed();
-  L.zeroed(d.st, static_cast<size_t>(n));
-  L.zeroed(d.pts0, H.pts.size());
-  L.zeroed(d.pts1, H.pts.size());
-  L.zeroed(d.paux, 3 * H.pts.size());
-  L.zeroed(d.poses0, H.poses.size());
-  L.zeroed(d.poses1, H.poses.size());
-  L.zeroed(d.part, static_cast<size_t>(part_off));
-  L.zeroed(d.sred, static_cast<size_t>(sred_off));
-  L.zeroed(d.A, static_cast<size_t>(a_off));
-  L.zeroed(d.dc, static_cast<size_t>(dc_off));
-  L.zeroed(d.dc64, static_cast<size_t>(dc_off));
-  L.zeroed(d.out_pts, H.pts.size());
-  L.zeroed(d.out_poses, H.poses.size());
-  L.zeroed(d.trace, static_cast<size_t>(n) * kTrace);
-  L.zeroed(d.bpart, bchunks.size());
+  auto plan = [&](int64_t pairs) {
+    const int64_t part_off = plan_chunks(b, H, pairs, h->opt.bchunk_pairs > 0 ? h->opt.bchunk_pairs : pairs);
+    return lay_out(b, H, part_off, sred_off, a_off, dc_off, pair_streams);
+  };
+  Layout L = plan(target);
+  if (use_default && target < kCoarseChunkPairs && L.total > memory_limit) L = plan(kCoarseChunkPairs);
+  Batch& d = b->dev;
+  d.n_windows = n;
+  d.red_blocks = H.red_first[n];
+  d.n_chunks = static_cast<int32_t>(H.chunks.size());
+  d.n_bchunks = static_cast<int32_t>(H.bchunks.size());
+  d.n_points = static_cast<int32_t>(H.pts.size());
+  d.n_poses = static_cast<int32_t>(H.poses.size() / 3);
+  d.n_cams = static_cast<int32_t>(H.cams.size() / 3);
+  d.loss = h->opt.loss;
+  d.fixed_iterations = h->opt.fixed_iterations;
+  d.max_rec = max_rec;
+  d.max_nc = max_nc;
   d.dbg_dp = nullptr;
   // shared-memory layout of the Schur kernel, sized for the batch's largest window. The key frames are staged
   // only while the layout leaves room for two workgroups per compute unit (80 KiB each); otherwise (large
@@ -1309,9 +1339,9 @@ int build_batch_impl(sba_handle* h, const sba_problem_view* problems, int32_t n,
 // Packs, uploads and (with `graph`) captures a batch; host allocation failures (the packing buffers are
 // page-locked) come back as a status, not as an exception through the C ABI.
 int build_batch(sba_handle* h, const sba_problem_view* problems, int32_t n, bool graph, const MemorySource& memory,
-                sba_batch** out, bool wait_upload = true) {
+                sba_batch** out, bool wait_upload = true, size_t memory_limit = SIZE_MAX) {
   try {
-    return build_batch_impl(h, problems, n, graph, wait_upload, memory, out);
+    return build_batch_impl(h, problems, n, graph, wait_upload, memory, memory_limit, out);
   } catch (const std::bad_alloc&) {
     *out = nullptr;
     return fail(h, SBA_E_INVALID, "out of host memory while packing");
@@ -1320,7 +1350,8 @@ int build_batch(sba_handle* h, const sba_problem_view* problems, int32_t n, bool
 
 // One window on the handle's stream, its device block taken from `memory`: packed, uploaded, solved with eager
 // launches (a different window shape on every call would need a new graph each time) and read back in place.
-int solve_one(sba_handle* h, const sba_problem_view* problem, sba_result* result, const MemorySource& memory) {
+int solve_one(sba_handle* h, const sba_problem_view* problem, sba_result* result, const MemorySource& memory,
+              size_t memory_limit = SIZE_MAX) {
   if (!h || !problem || !result) return fail(h, SBA_E_INVALID, "bad arguments to sba_solve");
   if (problem->num_points == 0 || problem->num_poses == 0 || problem->num_observations == 0) {
     result->status = SBA_E_EMPTY;
@@ -1330,7 +1361,7 @@ int solve_one(sba_handle* h, const sba_problem_view* problem, sba_result* result
   HIP_TRY(hipSetDevice(h->opt.device));
   TraceRange tr("SchurComplementBundlerGpu::solve");
   sba_batch* b = nullptr;
-  int rc = build_batch(h, problem, 1, false, memory, &b, false);  // sba_batch_read below waits for the stream
+  int rc = build_batch(h, problem, 1, false, memory, &b, false, memory_limit);  // sba_batch_read waits for the stream
   if (rc != SBA_OK) return rc;
   std::unique_ptr<sba_batch, int (*)(sba_batch*)> owned(b, free_batch);
   if ((rc = enqueue_solve(h, b, false)) != SBA_OK) return rc;
@@ -2112,22 +2143,14 @@ int sba_solve(sba_handle* h, const sba_problem_view* problem, sba_result* result
 }
 
 int sba_solve_noalloc(sba_handle* h, const sba_problem_view* problem, sba_result* result) {
-  const MemorySource scratch = [h](sba_batch*, size_t bytes, char** base) -> int {
+  return solve_one(h, problem, result, [h](sba_batch*, size_t bytes, char** base) -> int {
     if (!h->scratch) return fail(h, SBA_E_DEVICE, "the scratch array of sba_solve_noalloc is not set up");
     if (bytes > h->scratch_bytes)
       return fail(h, SBA_E_CAPACITY, "window needs " + std::to_string(bytes) + " bytes of device memory; "
                   "sba_solve_noalloc holds at most " + std::to_string(h->scratch_bytes) + " (use sba_solve)");
     *base = h->scratch;
     return SBA_OK;
-  };
-  int rc = solve_one(h, problem, result, scratch);
-  if (rc == SBA_E_CAPACITY && h->opt.chunk_pairs == 0) {
-    // small chunks trade memory for time (a record each): a window that does not fit with them may with coarse ones
-    h->opt.chunk_pairs = static_cast<int32_t>(kCoarseChunkPairs);
-    rc = solve_one(h, problem, result, scratch);
-    h->opt.chunk_pairs = 0;
-  }
-  return rc;
+  }, h ? h->scratch_bytes : 0);
 }
 
 }  // extern "C"

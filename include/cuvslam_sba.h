@@ -120,7 +120,9 @@ int sba_solve(sba_handle* h, const sba_problem_view* problem, sba_result* result
  * start at zero is cleared by a fill kernel, not a memset). The host side packs into ordinary host memory.
  * A window that needs more than the scratch holds returns SBA_E_CAPACITY and changes nothing (sba_solve takes any
  * size). Every handle on one GPU shares that GPU's array: calls that overlap on one GPU (several threads or
- * streams) race on it and must be serialized by the caller. Results are those of sba_solve. */
+ * streams) race on it and must be serialized by the caller. Results are those of sba_solve; a window that fits only
+ * without the default's small chunks (sba_options.chunk_pairs 0) is solved with chunks of 1024 pairs, and its results
+ * are those of sba_solve with chunk_pairs 1024 (sums in another order, the same but for rounding). */
 int sba_solve_noalloc(sba_handle* h, const sba_problem_view* problem, sba_result* result);
 
 /* Solves n independent windows of uneven size in one batch: every kernel of an LM iteration covers all

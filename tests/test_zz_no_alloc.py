@@ -54,3 +54,30 @@ def test_noalloc_rejects_a_window_beyond_its_scratch():
     assert solver.solve(want)
     rc, r, _, _ = solve_noalloc(solver, q)
     assert rc == _lib.SBA_OK and r.iterations == want.iterations
+
+
+def test_noalloc_takes_coarse_chunks_where_the_default_ones_do_not_fit():
+    # 38 free key frames make a record of 125 KB, and the default plan cuts these 2000 points into about 300 of them; 20
+    # cameras at the same place bring the observation streams to about 40 MB
+    p, _, _ = ca.scene.generate(seed=25, num_points=2000, num_keyframes=40, num_fixed_keyframes=2, max_iterations=3)
+    cameras, n = 20, p.num_observations
+    p.camera_from_rig = np.tile(p.camera_from_rig, (cameras, 1, 1))
+    p.camera_ids = np.repeat(np.arange(cameras), n).astype(np.int8)
+    p.observation_xys, p.pose_ids, p.point_ids = (np.tile(p.observation_xys, (cameras, 1)), np.tile(p.pose_ids, cameras),
+                                                  np.tile(p.point_ids, cameras))
+    p.observation_infos = np.tile(p.observation_infos, (cameras, 1, 1))
+    default, coarse = (ca.SchurComplementBundlerGpu(loss=ca.LOSS_HUBER, chunk_pairs=c) for c in (0, 1024))
+    counts = [s.batch([p]).info()["chunks"] for s in (default, coarse)]
+    assert (counts[0] - counts[1]) * 4 * (256 * 120 + 33 * 38) > 20 << 20  # what the coarse plan saves of records
+    want = p.copy()
+    assert coarse.solve(want)
+    rc, r, pts, poses = solve_noalloc(default, p)
+    assert rc == _lib.SBA_OK, default.last_error()
+    assert (r.iterations, r.accepted, r.last_cost_f64) == (want.iterations, want.accepted, want.last_cost_f64)
+    np.testing.assert_array_equal(pts, want.points)
+    np.testing.assert_array_equal(poses, want.rig_from_world)
+    rc, r, _, _ = solve_noalloc(coarse, p)  # an explicit size is kept, and this one fits
+    assert rc == _lib.SBA_OK and r.last_cost_f64 == want.last_cost_f64
+    tiles = ca.SchurComplementBundlerGpu(loss=ca.LOSS_HUBER, chunk_pairs=1)
+    rc, _, _, _ = solve_noalloc(tiles, p)  # this one does not
+    assert rc == _lib.SBA_E_CAPACITY
