@@ -19,8 +19,9 @@
 // blocks first would lose those digits (the gradients then differed by 1e-9 instead of 1e-12). A product is a pass over
 // these numbers instead of a new FP64 linearization of every observation. A conjugate-gradient iteration is four
 // launches: k_adj_hvp (y = H p), k_adj_update (x, r, and the Schur right-hand side), k_adj_reduced (the key-frame part,
-// dense) and k_adj_precond (z). Each workgroup owns whole points and adds over key frames into its own slot; the scalars
-// of an iteration are sums of one slot per workgroup, taken in slot order by every workgroup that needs them. 180k
+// dense) and k_adj_precond (z). Each workgroup owns whole points and adds over key frames into its own slot (atomically
+// in shared memory, so the last bits of two runs can differ); the scalars of an iteration are sums of one slot per
+// workgroup, taken in the same order by every workgroup that needs them. 180k
 // observations, 18 free key frames, microseconds per launch: 15.6 + 10.9 + 13.9 + 8.8 an iteration, 31.5 to assemble;
 // with a linearization of every observation per product (FP64 atomics on the points) and the vector algebra in
 // one workgroup, an iteration was seven launches of 47 + 15.5 + 12.6 + 15 + 42 + 15.5 + 15.5. The passes are bound by the
@@ -557,12 +558,15 @@ __global__ __launch_bounds__(1024) void k_adj_reduced(AdjData A) {
   __shared__ double sh[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n6 = A.n6;
   if (!INIT && *A.done) return;
-  auto sum = [&](double x) {  // over the workgroup, fixed order
+  auto wave_sums = [&](double x) {  // to sh, one per wavefront
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
     __syncthreads();
     if (lane == 0) sh[wave] = x;
     __syncthreads();
+  };
+  auto sum = [&](double x) {  // over the workgroup, fixed order
+    wave_sums(x);
     double s = 0.0;
     for (int k = 0; k < 16; ++k) s += sh[k];
     return s;
@@ -583,9 +587,10 @@ __global__ __launch_bounds__(1024) void k_adj_reduced(AdjData A) {
   red[tid] = e;
   double alpha = 0.0;
   if (!INIT) {
-    double py = 0.0;
-    for (int g = tid; g < A.slots; g += 1024) py += A.s_py[g];
-    py = sum(py);
+    // p.y in slot_sum's order, so that this step and its stop are those of k_adj_update to the last bit
+    static_assert(kAdjSlots <= kBlock && kBlock == 256, "one slot per thread of four wavefronts");
+    wave_sums(tid < A.slots ? A.s_py[tid] : 0.0);
+    const double py = (sh[0] + sh[1]) + (sh[2] + sh[3]);
     if (!(py > 0.0)) {  // workgroup-uniform
       if (tid == 0) *A.done = 1;
       return;
