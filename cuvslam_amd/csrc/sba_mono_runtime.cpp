@@ -6,7 +6,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <cstring>
-#include <new>
+#include <exception>
 #include <string>
 #include <thread>
 #include <vector>
@@ -82,7 +82,7 @@ int sba_mono_solve_batch(sba_handle* h, const sba_mono_window* windows, int32_t 
     else
       try {
         if (!pack_window(v, packs[i])) state[i] = 2;
-      } catch (const std::bad_alloc&) {  // must not leave a pool thread
+      } catch (const std::exception&) {  // allocation failures must not leave a pool thread
         state[i] = 3;
       }
   });

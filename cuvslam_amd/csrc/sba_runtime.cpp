@@ -15,6 +15,7 @@
 #include <condition_variable>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <functional>
 #include <memory>
 #include <mutex>
@@ -96,9 +97,9 @@ using pinned_vector = std::vector<T, PinnedAllocator<T>>;
 
 // Host threads kept by a handle: run(n, fn) calls fn(0) .. fn(n - 1), fn(0) on the calling thread, and returns when
 // all have returned. Threads are started on first need and end with the handle, so a solve does not pay for
-// thread creation. Between jobs a thread polls for the next one for up to kSpin before it sleeps: the packing
-// issues its phases back to back, and waking sleeping threads for each would cost more than the phases. Not
-// reentrant: fn must not call run().
+// thread creation; where the system gives no more, the calling thread makes the calls that have none. Between jobs
+// a thread polls for the next one for up to kSpin before it sleeps: the packing issues its phases back to back, and
+// waking sleeping threads for each would cost more than the phases. Not reentrant: fn must not call run().
 class HostPool {
  public:
   HostPool() = default;
@@ -117,20 +118,26 @@ class HostPool {
       fn(0);
       return;
     }
+    int have = n;  // calls that have a thread of their own
     {
       std::lock_guard<std::mutex> g(m_);
-      while (static_cast<int>(threads_.size()) < n - 1) {
-        const int id = static_cast<int>(threads_.size()) + 1;
-        const uint64_t seen = gen_.load();
-        threads_.emplace_back([this, id, seen] { worker(id, seen); });
+      try {
+        while (static_cast<int>(threads_.size()) < n - 1) {
+          const int id = static_cast<int>(threads_.size()) + 1;
+          const uint64_t seen = gen_.load();
+          threads_.emplace_back([this, id, seen] { worker(id, seen); });
+        }
+      } catch (const std::exception&) {  // no more threads: the calls left over run here
+        have = static_cast<int>(threads_.size()) + 1;
       }
       job_ = &fn;
-      job_n_ = n;
+      job_n_ = have;
       pending_.store(static_cast<int>(threads_.size()));
       gen_.fetch_add(1, std::memory_order_release);
     }
     wake_.notify_all();
     fn(0);
+    for (int k = have; k < n; ++k) fn(k);
     const auto t0 = std::chrono::steady_clock::now();
     while (pending_.load(std::memory_order_acquire) != 0) {
       if (std::chrono::steady_clock::now() - t0 > kSpin) {

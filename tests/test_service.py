@@ -40,3 +40,10 @@ def test_host_runtime_binds_every_stream_inside_its_block(target):
     out = subprocess.run([exe], capture_output=True, text=True, timeout=600)
     assert out.returncode == 0, out.stdout + out.stderr
     assert out.stdout.strip().splitlines()[-1].startswith("OK"), out.stdout
+
+
+def test_host_runtime_without_further_threads():
+    exe = build("runtime_no_threads_check")
+    out = subprocess.run([exe], capture_output=True, text=True, timeout=600)
+    assert out.returncode == 0, out.stdout + out.stderr
+    assert out.stdout.strip().splitlines()[-1].startswith("OK"), out.stdout
