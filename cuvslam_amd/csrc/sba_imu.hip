@@ -701,7 +701,7 @@ __global__ __launch_bounds__(kReducedThreads) void k_imu_reduced(Window w) {
 __global__ __launch_bounds__(kFactorThreads) void k_imu_factor(Window w) {
   using namespace sba_tiles;
   __shared__ double PT[(kMaxFree - 1) * 256];         // panel tiles of the current column, transposed
-  __shared__ double xt[256], yk[16], rdiag[16];
+  __shared__ double xt[256], yk[16];
   __shared__ double x[16 * kMaxFree];                 // right-hand side, then y, then the step (padded by tiles)
   __shared__ unsigned char nz[kMaxFree * kMaxFree];  // nz[i * nb + j], i >= j: tile (i, j) of L is not zero
   __shared__ int rows[kMaxFree];
@@ -734,7 +734,7 @@ __global__ __launch_bounds__(kFactorThreads) void k_imu_factor(Window w) {
       double4v t;
 #pragma unroll
       for (int v = 0; v < 4; ++v) t[v] = D[64 * v + lane];
-      const bool pos = factor_tile(t, xt, rdiag, lane);
+      const bool pos = factor_tile(t, xt, nullptr, lane);
       wave_lds_sync();
 #pragma unroll
       for (int v = 0; v < 4; ++v) D[64 * v + lane] = xt[64 * v + lane];
@@ -835,7 +835,7 @@ __global__ __launch_bounds__(kFactorThreads) void k_imu_factor(Window w) {
 __global__ __launch_bounds__(kFactorThreads) void k_imu_factor_lds(Window w) {
   using namespace sba_tiles;
   __shared__ double sm[kLdsTiles * 256];
-  __shared__ double xt[256], yk[16], rdiag[16], x[16 * kMaxFree];
+  __shared__ double xt[256], yk[16], x[16 * kMaxFree];
   __shared__ short slot[kMaxFree * (kMaxFree + 1) / 2];
   __shared__ int rows[2][kMaxFree], nrows[2];
   __shared__ int ok;
@@ -856,7 +856,7 @@ __global__ __launch_bounds__(kFactorThreads) void k_imu_factor_lds(Window w) {
   auto tile = [&](int i, int j) { return sm + 256 * slot[index(i, j)]; };
   // wavefront 0: factor diagonal tile k (its value in t), y_k = X b_k, the panel rows of column k
   auto pivot = [&](int k, double4v t) {
-    const bool pos = factor_tile(t, xt, rdiag, lane);
+    const bool pos = factor_tile(t, xt, nullptr, lane);
     const bool has = lane > k && lane < nb && slot[index(min(lane, nb - 1), min(k, min(lane, nb - 1)))] >= 0;
     const unsigned long long mask = __ballot(has);
     if (has) rows[k & 1][__popcll(mask & ((1ull << lane) - 1))] = lane;

@@ -173,7 +173,7 @@ __device__ __forceinline__ double4v staged_update(double4v c, const double* p, c
 // Shared memory of factor_block, in doubles: diagonal tiles, their inverses transposed, the current panel, the
 // off-diagonal tiles of A and of X, the right-hand side.
 constexpr int kFbDg = 0, kFbXT = kFbDg + 4 * 256, kFbP = kFbXT + 4 * 256, kFbU = kFbP + 4 * 256, kFbX = kFbU + 6 * 256,
-              kFbVec = kFbX + 6 * 256, kFbY = kFbVec + kLB, kFbIdg = kFbY + kLB, kFbWords = kFbIdg + kLB;
+              kFbVec = kFbX + 6 * 256, kFbY = kFbVec + kLB, kFbWords = kFbY + kLB;
 
 // pair index of tile (J, I), J < I < 4: 0 (0,1) 1 (0,2) 2 (0,3) 3 (1,2) 4 (1,3) 5 (2,3)
 __device__ __forceinline__ int pair_of(int J, int I) { return J == 0 ? I - 1 : (J == 1 ? I + 1 : 5); }
@@ -194,7 +194,7 @@ __device__ bool factor_block(double* sm, int* flag, double* Xg, double* rhs, int
   double* sP = sm + kFbP;
   double* sU = sm + kFbU;
   double* sX = sm + kFbX;
-  double *vec = sm + kFbVec, *ys = sm + kFbY, *idg = sm + kFbIdg;
+  double *vec = sm + kFbVec, *ys = sm + kFbY;
   const int lane = tid & 63, li = lane >> 4, lj = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   auto forward = [&](int K) {  // y_K = X_KK e_K, lane l holds y_K[l % 16]
@@ -218,7 +218,7 @@ __device__ bool factor_block(double* sm, int* flag, double* Xg, double* rhs, int
 #pragma unroll
         for (int v = 0; v < 4; ++v) dt[v] = tk[64 * v + lane];
         if (K >= 0) dt = tile_update(dt, sP + 256 * (K + 1), sP + 256 * (K + 1), lane);
-        if (!factor_tile(dt, sXT + 256 * (K + 1), idg + 16 * (K + 1), lane) && lane == 0) *flag = 1;
+        if (!factor_tile(dt, sXT + 256 * (K + 1), nullptr, lane) && lane == 0) *flag = 1;
       }
       __syncthreads();
     }
@@ -336,7 +336,10 @@ __global__ __launch_bounds__(256) void k_lfirst(Batch b, int w) {
 // solve, and takes e_i -= L_ik y_k. The first workgroup, block (k + 1, k + 1), goes on to factor its block
 // (factor_block), so the next step starts with its inverse: one launch per block column, bound by that workgroup's serial
 // chain. Order 1194: 24 us per block column, against 45 us with separate diagonal, panel and trailing launches (24 + 11
-// + 10); order 336: 23.5 against 43.
+// + 10); order 336: 23.5 against 43. In a large system the trailing updates take over, where the recomputed panels cost
+// what the launches save: gather, factor and backward solve per iteration, here against separate launches, order 2394
+// 1.38 against 2.36 ms, 3594 2.85 against 4.20, 4794 5.16 against 6.64, 6114 (1020 key frames, the most a window may hold
+// is 1024) 10.1 against 10.3. So one rule serves every order.
 __global__ __launch_bounds__(256) void k_lstep(Batch b, int w, int k) {
   __shared__ double sm[3 * 16 * kTs];
   __shared__ double sy[kLB], sred[4 * kLB];

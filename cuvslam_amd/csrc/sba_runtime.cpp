@@ -835,14 +835,17 @@ int check_streams(sba_handle* h, const Batch& d) {
 // Pairs of work per chunk when the options leave it open. A chunk is one workgroup that runs its tiles one after
 // another, and two workgroups fit on a compute unit, so up to 512 chunks run at once: below 1024 x 512 pairs a chunk
 // takes only its share of those, down to a single tile (a chunk never has less), as long as the records of all chunks
-// stay within kRecordBytes (`record_work`: the sum over windows of pairs x record bytes; a record is written and read
-// back once per iteration). Above, at least 1024 pairs, so that a chunk's record stays small against its work, and
-// about 32 chunks per compute unit, so that the dispatcher balances uneven windows. Measured, microseconds of the Schur
-// kernel at 1024 pairs per chunk -> at the share: 13.9k pairs 68 -> 15 (one tile per chunk), 53k pairs on 56 free key
-// frames 235 -> 41, 582k pairs 61 (the same; 512 pairs 73, 2048 pairs 96). 6.7M pairs in 128 windows: whole iterations
-// 1.29 ms at 1024, 1.28 at 1536 to 2048, 1.36 at 512 or 3072. Records of 118 KB (38 free key frames): 153k pairs 1.83 ms
-// per solve at one tile per chunk (79 MB of records), 1.75 at 384 pairs (40 MB), 2.07 at 1024; 383k pairs 2.64, 2.15 at
-// 768 (49 MB), 2.32.
+// of windows with at most kMaxFreePoses free key frames stay within kRecordBytes (`record_work`: the sum over these
+// windows of pairs x record bytes; a record is written and read back once per iteration). Above, at least 1024 pairs,
+// so that a chunk's record stays small against its work, and about 32 chunks per compute unit, so that the dispatcher
+// balances uneven windows. Measured, microseconds of the Schur kernel at 1024 pairs per chunk -> at the share: 13.9k
+// pairs 68 -> 15 (one tile per chunk), 53k pairs on 56 free key frames 235 -> 41, 582k pairs 61 (the same; 512 pairs
+// 73, 2048 pairs 96). 6.7M pairs in 128 windows: whole iterations 1.29 ms at 1024, 1.28 at 1536 to 2048, 1.36 at 512 or
+// 3072. Records of 118 KB (38 free key frames): 153k pairs 1.83 ms per solve at one tile per chunk (79 MB of records),
+// 1.75 at 384 pairs (40 MB), 2.07 at 1024; 383k pairs 2.64, 2.15 at 768 (49 MB), 2.32. Larger windows' records hold
+// only the key frames that a chunk stages, and their share pays without a bound: 347k pairs on 99 free key frames 3.37
+// ms per solve at the share (678 pairs), 3.21 at 256, 3.89 at 1024; 502k on 199, 5.41 at 979, 5.32 at 512, 5.54 at
+// 1024; 87k on 56, 1.54 at 169, 2.42 at 1024.
 constexpr int64_t kCoarseChunkPairs = 1024;
 int64_t default_chunk_pairs(int64_t total_pairs, double record_work) {
   constexpr int64_t kResident = 512;
@@ -1149,8 +1152,8 @@ int64_t plan_chunks(sba_batch* b, HostPack& H, int64_t target, int64_t btarget) 
   return part_off;
 }
 
-// The device block of the planned batch: `part`, `sred`, `a` and `dc` elements of records, reduced records, mapped windows'
-// FP64 systems and steps; `pair_streams`: pairs have their own copy of their first observation.
+// The device block of the planned batch: `part`, `sred`, `a` and `dc` elements of records, reduced records, FP64 systems
+// of mapped windows and steps; `pair_streams`: pairs have their own copy of their first observation.
 Layout lay_out(sba_batch* b, const HostPack& H, int64_t part, int64_t sred, int64_t a, int64_t dc, bool pair_streams) {
   Batch& d = b->dev;
   Layout L;

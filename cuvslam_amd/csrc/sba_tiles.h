@@ -90,8 +90,8 @@ __device__ __forceinline__ void rows_of(double x, double (&r)[4]) {
 //   U_v = L_vv^-1 A_v and X_v = L_vv^-1 I_v by forward substitution, every lane with its column's four rows;
 //   A -= U_v^T U_v and I -= U_v^T X_v, one matrix instruction each: the panel is at once the B operand and the A operand
 //   of its transpose.
-// On return t holds U (zero below the diagonal), X^T is written to xt (row-major) and 1 / U_ii to rdiag. False on a
-// pivot that is not positive and finite (the values are then dropped by the callers).
+// On return t holds U (zero below the diagonal), X^T is written to xt (row-major) and, unless rdiag is null, 1 / U_ii to
+// rdiag. False on a pivot that is not positive and finite (the values are then dropped by the callers).
 //
 // A serial chain bounds it: 16 reciprocal square roots with a few dependent FMAs each, and one matrix instruction per
 // panel between them; the substitutions run beside the chain of their own block. Measured alone on one wavefront: 1.07 us;
@@ -146,7 +146,7 @@ __device__ inline bool factor_tile(double4v& t, double* xt, double* rdiag, int l
   for (int v = 0; v < 4; ++v) {
     t[v] = u[v];
     xt[16 * col + 4 * v + row] = x[v];
-    if (4 * v + row == col) rdiag[col] = x[v];
+    if (rdiag && 4 * v + row == col) rdiag[col] = x[v];
   }
   return ok;
 }

@@ -1,5 +1,5 @@
 """The blocked factor of windows with more than 40 free key frames at its block edges: reduced systems whose order
-leaves a last 64-row block of 2, 8, 54, 56, 62 and 64 rows."""
+leaves a last 64-row block of 2, 8, 54, 58, 60, 62 and 64 rows."""
 import numpy as np
 import pytest
 
