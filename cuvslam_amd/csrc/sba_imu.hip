@@ -831,7 +831,7 @@ __global__ __launch_bounds__(kFactorThreads) void k_imu_factor(Window w) {
 // in global memory between the barriers of every column was most of the time. After the panel step a slot holds
 // L_ik^T, the operand of the trailing updates, instead of A_ik. Wavefront 0 updates and factors the next diagonal
 // tile while the others run the trailing updates, so a column is two barriers and wavefront 0's chain bounds it:
-// 19 free key frames on 2-frame tracks (37 tiles) 72 us, 110 with the tiles in global memory; 9 free key frames 38 us.
+// 19 free key frames on 2-frame tracks (37 tiles) 70 us, 110 with the tiles in global memory; 9 free key frames 36 us.
 __global__ __launch_bounds__(kFactorThreads) void k_imu_factor_lds(Window w) {
   using namespace sba_tiles;
   __shared__ double sm[kLdsTiles * 256];
@@ -1168,7 +1168,7 @@ hipError_t imu_model(const Window& w, hipStream_t s) {
 hipError_t imu_step(const Window& w, hipStream_t s) {
   if (w.P > 0) hipLaunchKernelGGL(k_imu_point_inv, dim3(blocks(w.P, kThreads / kPointLanes)), dim3(kThreads), 0, s, w);
   if (w.n > 0) hipLaunchKernelGGL(k_imu_reduced, dim3(w.nblocks + w.n), dim3(kReducedThreads), 0, s, w);
-  // Tiles in shared memory whenever they fit: it is the faster one at every size (72 against 110 us at 37 tiles). Both
+  // Tiles in shared memory whenever they fit: it is the faster one at every size (70 against 110 us at 37 tiles). Both
   // set chol_ok; without free key frames the first has no tile to start from.
   if (w.n > 0 && w.nslots <= kLdsTiles)
     hipLaunchKernelGGL(k_imu_factor_lds, dim3(1), dim3(kFactorThreads), 0, s, w);

@@ -831,7 +831,7 @@ __global__ __launch_bounds__(256) void k_reduce(Batch b) {
 // Two barriers per tile column. Wavefront 0's chain bounds it: a panel product, an update and a 16 x 16 factor per column;
 // that it forms the one panel tile it needs itself takes the wait for the other wavefronts' panel out of the chain.
 // Backward substitution U x = y per tile column: wavefront 0 forms r_K -= U_{K,K+1} x_{K+1} and x_K = X_KK^T r_K while
-// the tiles' owners apply x_{K+1} to the rows above; one barrier per column. 28 free key frames (11 tile columns): 58 us,
+// the tiles' owners apply x_{K+1} to the rows above; one barrier per column. 28 free key frames (11 tile columns): 57 us,
 // 66 with every panel tile formed by its owner and the backward row updates in one chain with x_K.
 // (Golub & Van Loan, Matrix Computations, 4.2.4 block Cholesky and 3.1 triangular systems.)
 // ---------------------------------------------------------------------------------------------------------

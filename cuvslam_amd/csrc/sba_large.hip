@@ -335,8 +335,8 @@ __global__ __launch_bounds__(256) void k_lfirst(Batch b, int w) {
 // transposed, in the unused upper triangle (block (k, i); the lower A_ik is still read by others) for the backward
 // solve, and takes e_i -= L_ik y_k. The first workgroup, block (k + 1, k + 1), goes on to factor its block
 // (factor_block), so the next step starts with its inverse: one launch per block column, bound by that workgroup's serial
-// chain. Order 1194: 24 us per block column, against 45 us with separate diagonal, panel and trailing launches (24 + 11
-// + 10); order 336: 23.5 against 43. In a large system the trailing updates take over, where the recomputed panels cost
+// chain. Order 1194: 23 us per block column, against 45 us with separate diagonal, panel and trailing launches (24 + 11
+// + 10); order 336: 22 against 43. In a large system the trailing updates take over, where the recomputed panels cost
 // what the launches save: gather, factor and backward solve per iteration, here against separate launches, order 2394
 // 1.38 against 2.36 ms, 3594 2.85 against 4.20, 4794 5.16 against 6.64, 6114 (1020 key frames, the most a window may hold
 // is 1024) 10.1 against 10.3. So one rule serves every order.
